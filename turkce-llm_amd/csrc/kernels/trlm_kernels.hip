@@ -2,6 +2,7 @@
 // Built with: hipcc --genco --offload-arch=gfx950 -O3
 //             -Xclang -target-feature -Xclang -packed-fp32-ops
 #include "gemm.hip"
+#include "gemm_split.hip"
 #include "rowops.hip"
 #include "attention.hip"
 #include "decode.hip"

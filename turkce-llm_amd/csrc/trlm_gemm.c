@@ -28,11 +28,14 @@
 enum { L_NN = 0, L_NT = 1, L_TN = 2 };
 static const char* LAYOUT_NAME[4] = { "nn", "nt", "tn", "tt" };
 
-/* Aligned tile variants (gemm.hip): name suffix, tile rows/cols, k step. */
+/* Aligned tile variants: name suffix, tile rows/cols, k step.  128x128,
+ * 64x128_k32 and 64x64_k32 form their products on the bf16 matrix cores from
+ * exact three-way splits (gemm_split.hip); the others, which only
+ * trlm_gemm_force selects, use the fp32 matrix cores (gemm.hip). */
 typedef struct TileDef { const char* name; int bm, bn, bk; } TileDef;
 enum { T_256x128, T_128x256, T_128x128, T_128x128_K32, T_64x128, T_64x128_K32, T_64x64, T_64x64_K32, T_COUNT };
 static const TileDef TILES[T_COUNT] = {
-    { "256x128", 256, 128, 16 }, { "128x256", 128, 256, 16 }, { "128x128", 128, 128, 16 },
+    { "256x128", 256, 128, 16 }, { "128x256", 128, 256, 16 }, { "128x128", 128, 128, 32 },
     { "128x128_k32", 128, 128, 32 }, { "64x128", 64, 128, 16 }, { "64x128_k32", 64, 128, 32 },
     { "64x64", 64, 64, 16 }, { "64x64_k32", 64, 64, 32 },
 };
@@ -46,7 +49,7 @@ struct TrlmGemm {
     hipFunction_t ku[4];
     hipFunction_t reduce;
     hipFunction_t reduce4;   /* four columns per thread, for 16-byte aligned operands */
-    hipFunction_t glu;   /* k_gemm_nn_64x64_k32_glu */
+    hipFunction_t glu, glu128;   /* SwiGLU epilogue: k_gemm_nn_64x64_k32_glu, k_swiglu_gemm_128x128 */
     hipDeviceptr_t ws;
     u64 ws_floats;
     char last[48];
@@ -72,6 +75,7 @@ TrlmGemm* trlm_gemm_create(HipCtx* ctx) {
     e->reduce = hip_get_kernel(ctx, "k_gemm_splitk_reduce");
     e->reduce4 = hip_get_kernel(ctx, "k_gemm_splitk_reduce4");
     e->glu = hip_get_kernel(ctx, "k_gemm_nn_64x64_k32_glu");
+    e->glu128 = hip_get_kernel(ctx, "k_swiglu_gemm_128x128");
     trlm_noalloc_setup(ctx->device);
     return e;
 }
@@ -140,38 +144,43 @@ static int auto_splits(long long tiles, int K) {
 /* Plan model: the tiles' workgroups are spread evenly over the 256 CUs, so
  * the busiest CU runs n = ceil(workgroups / 256) of them, `occ` at a time
  * (the variant's resident workgroups per CU).  A CU with c resident
- * workgroups runs at cu_rate(c) of its steady-state rate (one resident
- * 4-wave workgroup cannot hide its own load latency), and each variant has
- * its own steady-state efficiency.  The last resident batch adds an
- * imbalance term proportional to a workgroup's duration.  Split-K adds the
- * partials' round trip through HBM plus the reduction launch.  Constants
- * fitted to MI355X timings of every variant/split on the model's GEMMs at
- * 512-8192 rows (within 0.6 % of the per-shape best over those 45 shapes). */
-typedef struct PlanTile { int tile; int occ; double eff; } PlanTile;
+ * workgroups runs at cu_rate of the variant's steady-state rate (a lone
+ * workgroup's split and LDS phases leave its matrix cores idle, several
+ * workgroups' phases overlap).  The last resident batch adds an imbalance
+ * term proportional to a workgroup's duration, and no plan is faster than
+ * the chip's sustained rate (the matrix cores' clock falls under load).
+ * Split-K adds the partials' round trip through HBM plus the reduction
+ * launch.  Constants fitted to MI355X timings of the three split-product
+ * variants and every split on the model's GEMMs at 300-8192 rows and five
+ * others (within 0.8 % of the per-shape best over those 70 shapes). */
+typedef struct PlanTile { int tile; int occ; double rate, lone; } PlanTile;
 static const PlanTile PLAN_TILES[] = {
-    { T_128x128, 3, 1.047 }, { T_128x256, 2, 0.977 }, { T_256x128, 2, 1.008 },
-    { T_64x128_K32, 2, 0.955 }, { T_64x64_K32, 4, 0.992 },
+    { T_128x128, 3, 0.820e12, 0.781 }, { T_64x128_K32, 4, 0.627e12, 0.450 }, { T_64x64_K32, 5, 0.644e12, 0.662 },
 };
 static const int PLAN_SPLITS[] = { 1, 2, 3, 4, 6, 7, 8, 12, 16, 24, 32 };
-#define PLAN_CU_FLOPS 0.6e12     /* per-CU steady-state fp32 MFMA rate, FLOP/s */
-#define PLAN_SPLIT_BW 1.63e12    /* effective bytes/s of the partials' round trip */
-#define PLAN_SPLIT_FIXED 1.25e-6 /* reduction launch, s */
-#define PLAN_TAIL 0.075          /* last-round imbalance, in resident-batch durations */
+#define PLAN_CAP_FLOPS 227e12    /* the chip's sustained rate, FLOP/s */
+#define PLAN_SPLIT_BW 3.06e12    /* effective bytes/s of the partials' round trip */
+#define PLAN_SPLIT_FIXED 1.91e-6 /* reduction launch, s */
+#define PLAN_TAIL 0.123          /* last-round imbalance, in resident-batch durations */
 
-static double cu_rate(int c) { return c <= 1 ? 0.916 : 1.0; }
+static double cu_rate(const PlanTile* pt, long long c) {
+    return pt->lone + (1.0 - pt->lone) * (double)(c - 1) / (pt->occ - 1);
+}
 
 static double plan_cost(const PlanTile* pt, int M, int N, int K, u32 batch, int splits) {
     const TileDef* td = &TILES[pt->tile];
     double wg = (double)cdiv(M, td->bm) * cdiv(N, td->bn) * batch * splits;
     int kch = splits > 1 ? cdiv(cdiv(K, splits), KCHUNK_ALIGN) * KCHUNK_ALIGN : K;
     long long n = (long long)((wg + CUS - 1) / CUS);
-    double w = 2.0 * td->bm * td->bn * (double)kch / (pt->eff * PLAN_CU_FLOPS);
-    long long full = n / pt->occ, rest = n % pt->occ;
-    double t = (double)full * pt->occ * w / cu_rate(pt->occ);
-    if (rest) t += (double)rest * w / cu_rate((int)rest);
+    double flops = 2.0 * td->bm * td->bn * (double)kch;
+    double w = flops / pt->rate;
+    long long full = n / pt->occ, rest = n % pt->occ, last = n < pt->occ ? n : pt->occ;
+    double t = (double)full * pt->occ * w;
+    if (rest) t += (double)rest * w / cu_rate(pt, rest);
     /* workgroups of one resident batch finish unevenly: long workgroups
      * leave CUs idle at the end, which more, shorter ones even out */
-    t += PLAN_TAIL * pt->occ * w / cu_rate((int)(n < pt->occ ? n : pt->occ));
+    t += PLAN_TAIL * (double)last * w / cu_rate(pt, last);
+    if (t < wg * flops / PLAN_CAP_FLOPS) t = wg * flops / PLAN_CAP_FLOPS;
     if (splits > 1) t += (splits + 1) * (double)M * N * 4.0 / PLAN_SPLIT_BW + PLAN_SPLIT_FIXED;
     return t;
 }
@@ -277,11 +286,16 @@ i32 trlm_gemm_ws(TrlmGemm* e, i32 trans_a, i32 trans_b, hipDeviceptr_t A, hipDev
         p.A = (const float*)A; p.B = (const float*)B; p.C = (float*)C; p.bias = (const float*)bias;
         p.M = M; p.N = N; p.K = K; p.lda = lda; p.ldb = ldb; p.ldc = ldc; p.ldr = ldr;
         p.splits = 1; p.kchunk = K; p.alpha = alpha; p.beta = 0.0f;
-        p.tiles_m = cdiv(M, 64); p.tiles_n = cdiv(N, 64);
+        /* the 128-wide tile where F holds whole half tiles and the plan
+         * model finds it the faster of the two */
+        const int wide = x->glu_F % 64 == 0 && plan_cost(&PLAN_TILES[0], M, N, K, 1, 1) <
+                                                   plan_cost(&PLAN_TILES[2], M, N, K, 1, 1);
+        const int tile = wide ? 128 : 64;
+        p.tiles_m = cdiv(M, tile); p.tiles_n = cdiv(N, tile);
         p.glu_h = (float*)x->glu_h; p.glu_F = x->glu_F;
-        snprintf(e->last, sizeof(e->last), "k_gemm_nn_64x64_k32_glu");
+        snprintf(e->last, sizeof(e->last), wide ? "k_swiglu_gemm_128x128" : "k_gemm_nn_64x64_k32_glu");
         e->last_splits = 1;
-        launch(e->glu, &p, 1);
+        launch(wide ? e->glu128 : e->glu, &p, 1);
         return 0;
     }
     if (csum && (batch != 1 || trans_b)) {
