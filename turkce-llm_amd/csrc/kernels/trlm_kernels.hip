@@ -3,6 +3,7 @@
 //             -Xclang -target-feature -Xclang -packed-fp32-ops
 #include "gemm.hip"
 #include "gemm_split.hip"
+#include "gemm_small.hip"
 #include "rowops.hip"
 #include "attention.hip"
 #include "decode.hip"

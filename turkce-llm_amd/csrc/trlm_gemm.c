@@ -49,6 +49,8 @@ struct TrlmGemm {
     hipFunction_t ku[4];
     hipFunction_t reduce;
     hipFunction_t reduce4;   /* four columns per thread, for 16-byte aligned operands */
+    hipFunction_t small[2][3];   /* k_smallgemm_<layout>[_u]: 32x32 tiles, k shared out over a workgroup's waves */
+    hipFunction_t small_glu;
     hipFunction_t glu, glu128;   /* SwiGLU epilogue: k_gemm_nn_64x64_k32_glu, k_swiglu_gemm_128x128 */
     hipDeviceptr_t ws;
     u64 ws_floats;
@@ -72,6 +74,13 @@ TrlmGemm* trlm_gemm_create(HipCtx* ctx) {
         snprintf(name, sizeof(name), "k_gemm_%s_64x64_u", LAYOUT_NAME[l]);
         e->ku[l] = hip_get_kernel(ctx, name);
     }
+    for (int l = 0; l < 3; l++)
+        for (int u = 0; u < 2; u++) {
+            snprintf(name, sizeof(name), "k_smallgemm_%s%s", LAYOUT_NAME[l], u ? "_u" : "");
+            e->small[u][l] = hip_get_kernel(ctx, name);
+        }
+    snprintf(name, sizeof(name), "k_smallgemm_%s_glu", LAYOUT_NAME[L_NN]);
+    e->small_glu = hip_get_kernel(ctx, name);
     e->reduce = hip_get_kernel(ctx, "k_gemm_splitk_reduce");
     e->reduce4 = hip_get_kernel(ctx, "k_gemm_splitk_reduce4");
     e->glu = hip_get_kernel(ctx, "k_gemm_nn_64x64_k32_glu");
@@ -152,10 +161,12 @@ static int auto_splits(long long tiles, int K) {
  * Split-K adds the partials' round trip through HBM plus the reduction
  * launch.  Constants fitted to MI355X timings of the three split-product
  * variants and every split on the model's GEMMs at 300-8192 rows and five
- * others (within 0.8 % of the per-shape best over those 70 shapes). */
-typedef struct PlanTile { int tile; int occ; double rate, lone; } PlanTile;
+ * others (within 0.8 % of the per-shape best over those 80 shapes). */
+typedef struct PlanTile { int tile; int occ; double rate, lone, start; } PlanTile;
 static const PlanTile PLAN_TILES[] = {
-    { T_128x128, 3, 0.820e12, 0.781 }, { T_64x128_K32, 4, 0.627e12, 0.450 }, { T_64x64_K32, 5, 0.644e12, 0.662 },
+    { T_128x128, 3, 0.820e12, 0.781, 2e-6 },
+    { T_64x128_K32, 4, 0.627e12, 0.450, 0 },
+    { T_64x64_K32, 5, 0.644e12, 0.662, 0 },
 };
 static const int PLAN_SPLITS[] = { 1, 2, 3, 4, 6, 7, 8, 12, 16, 24, 32 };
 #define PLAN_CAP_FLOPS 227e12    /* the chip's sustained rate, FLOP/s */
@@ -181,6 +192,7 @@ static double plan_cost(const PlanTile* pt, int M, int N, int K, u32 batch, int 
      * leave CUs idle at the end, which more, shorter ones even out */
     t += PLAN_TAIL * (double)last * w / cu_rate(pt, last);
     if (t < wg * flops / PLAN_CAP_FLOPS) t = wg * flops / PLAN_CAP_FLOPS;
+    t += pt->start;   /* first loads and last stores of a workgroup, over the smallest tile's */
     if (splits > 1) t += (splits + 1) * (double)M * N * 4.0 / PLAN_SPLIT_BW + PLAN_SPLIT_FIXED;
     return t;
 }
@@ -189,18 +201,19 @@ static void select_plan(int M, int N, int K, u32 batch, int* tile, int* splits) 
     double best = 0.0;
     *tile = T_128x128;
     *splits = 1;
-    /* Decode-sized products (M <= 128 rows, few tiles): each workgroup's
-     * k loop is latency-bound (~1 us per 32-deep step), so split K down to
-     * 64-deep chunks over up to 8 partitions, one workgroup per CU at most.
-     * Measured on MI355X at M = 64: QKV 12.8 -> 9.0 us, attention-out 11.8
-     * -> 8.6, gate_up 12.4 -> 8.2, down (K = 1024) 12.6 -> 10.4, reduction
-     * included. */
-    if (M <= 128 && batch == 1) {
+    /* Products of few tiles with one side of at most 128: each workgroup's k
+     * loop is latency-bound (0.75 us per 32-deep step alone on its CU), so
+     * split K down to 64-deep chunks over up to 8 partitions, 128-deep up to
+     * 16 and 256-deep beyond, two workgroups per CU at most.  Measured on
+     * MI355X against at most 8: 17x1374x7742 35.3 -> 27.2 us (16). */
+    if ((M <= 128 || N <= 128) && batch == 1) {
         long long tiles = (long long)cdiv(M, 64) * cdiv(N, 64);
         if (tiles < 128) {
             long long smax = K / 64;
             if (smax > 8) smax = 8;
-            if (smax > CUS / tiles) smax = CUS / tiles;
+            if (smax < K / 128) smax = K / 128 < 16 ? K / 128 : 16;
+            if (smax < K / 256) smax = K / 256;
+            if (smax > 2 * CUS / tiles) smax = 2 * CUS / tiles;
             *tile = T_64x64_K32;
             for (size_t j = 0; j < sizeof(PLAN_SPLITS) / sizeof(PLAN_SPLITS[0]); j++)
                 if (PLAN_SPLITS[j] <= smax) *splits = PLAN_SPLITS[j];
@@ -220,6 +233,26 @@ static void select_plan(int M, int N, int K, u32 batch, int* tile, int* splits) 
         }
 }
 
+/* Products of few tiles (gemm_small.hip, reported as the tile 32x32): one
+ * 32x32 tile per workgroup, k shared out over its waves.  Up to two tiles per
+ * CU, measured on MI355X against the planned tile (us): 64x1152x384 5.8 / 8.0,
+ * 128x2048x384 (256 tiles) 6.1 / 9.9, 512x384x384 (192) 6.0 / 11.9,
+ * 512x1024x384 (512) 9.9 / 10.8, but 512x1152x384 (576) 12.4 / 12.2; with less
+ * than 96 k up to one tile per CU (384x1152x64, 432 tiles: 5.2 / 4.9).  Up to
+ * 768 k, 1152 where neither side is at most 128 (512x384x1024 11.0 / 13.4,
+ * 358x137x1099 12.9 / 14.6, but 64x384x1024, which select_plan splits into
+ * more partitions, 10.8 / 9.4).  Unaligned operands, whose other kernel has no
+ * split: up to four tiles per CU (1000x701x333 16.3 / 19.8, but 2001x1001x333
+ * 34.8 / 30.1). */
+static int small_gemm(int M, int N, int K, u32 batch, int aligned) {
+    const long long tiles = (long long)cdiv(M, 32) * cdiv(N, 32);
+    const int most = !aligned ? 4 * CUS : K >= 96 ? 2 * CUS : CUS;
+    return batch == 1 && K <= (M > 128 && N > 128 ? 1152 : 768) && tiles <= most;
+}
+
+/* How many ways its waves share out k: up to four, 32 k at a time. */
+static int small_splits(int K) { return K > 96 ? 4 : K > 32 ? cdiv(K, 32) : 1; }
+
 const char* trlm_gemm_plan(i32 trans_a, i32 trans_b, i32 M, i32 N, i32 K, u32 batch, i32* splits) {
     static __thread char name[48];
     int layout = trans_a ? (trans_b ? 3 : L_TN) : (trans_b ? L_NT : L_NN);
@@ -227,6 +260,9 @@ const char* trlm_gemm_plan(i32 trans_a, i32 trans_b, i32 M, i32 N, i32 K, u32 ba
     if (layout == 3) {
         snprintf(name, sizeof(name), "k_gemm_tt_64x64_u");
         sp = 1;
+    } else if (small_gemm(M, N, K, batch ? batch : 1, 1)) {
+        snprintf(name, sizeof(name), "k_gemm_%s_32x32", LAYOUT_NAME[layout]);
+        sp = small_splits(K);
     } else {
         select_plan(M, N, K, batch ? batch : 1, &tile, &sp);
         if (sp > 1) sp = cdiv(K, cdiv(cdiv(K, sp), KCHUNK_ALIGN) * KCHUNK_ALIGN);
@@ -288,6 +324,14 @@ i32 trlm_gemm_ws(TrlmGemm* e, i32 trans_a, i32 trans_b, hipDeviceptr_t A, hipDev
         p.splits = 1; p.kchunk = K; p.alpha = alpha; p.beta = 0.0f;
         /* the 128-wide tile where F holds whole half tiles and the plan
          * model finds it the faster of the two */
+        if (small_gemm(M, N, K, 1, 1)) {
+            p.tiles_m = cdiv(M, 32); p.tiles_n = N / 32;
+            p.glu_h = (float*)x->glu_h; p.glu_F = x->glu_F;
+            snprintf(e->last, sizeof(e->last), "k_gemm_%s_32x32_glu", LAYOUT_NAME[L_NN]);
+            e->last_splits = small_splits(K);
+            launch(e->small_glu, &p, 1);
+            return 0;
+        }
         const int wide = x->glu_F % 64 == 0 && plan_cost(&PLAN_TILES[0], M, N, K, 1, 1) <
                                                    plan_cost(&PLAN_TILES[2], M, N, K, 1, 1);
         const int tile = wide ? 128 : 64;
@@ -329,6 +373,13 @@ i32 trlm_gemm_ws(TrlmGemm* e, i32 trans_a, i32 trans_b, hipDeviceptr_t A, hipDev
     int layout = trans_a ? (trans_b ? 3 : L_TN) : (trans_b ? L_NT : L_NN);
     int aligned = layout != 3 && aligned16(A) && aligned16(B) && (lda % 4 == 0) && (ldb % 4 == 0) &&
                   (batch == 1 || ((sA % 4 == 0) && (sB % 4 == 0)));
+    if (layout != 3 && !stats && e->force_tile < 0 && e->force_splits == 0 && small_gemm(M, N, K, batch, aligned)) {
+        p.tiles_m = cdiv(M, 32); p.tiles_n = cdiv(N, 32);
+        snprintf(e->last, sizeof(e->last), "k_gemm_%s_32x32%s", LAYOUT_NAME[layout], aligned ? "" : "_u");
+        e->last_splits = small_splits(K);
+        launch(e->small[!aligned][layout], &p, 1);
+        return 0;
+    }
     if (!aligned) {
         p.tiles_m = cdiv(M, 64); p.tiles_n = cdiv(N, 64);
         snprintf(e->last, sizeof(e->last), "k_gemm_%s_64x64_u", LAYOUT_NAME[layout]);
