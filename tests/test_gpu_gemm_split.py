@@ -9,7 +9,7 @@ parts, six products on the bf16 matrix cores.
     rounding would leave in all rows alike is no more than the fp32 variant's;
   - infinities, NaN and magnitudes that bf16 rounds to infinity come out as
     fp32 gives them, and padding past N never reaches C;
-  - the SwiGLU epilogue of the 128-wide tile equals the unfused path.
+  - the SwiGLU epilogues agree with the oracle through the decoder's prefill.
 """
 import numpy as np
 import pytest
@@ -89,6 +89,35 @@ def test_edges(dev, tile, ta, tb, M, N, K, splits):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0), (1, 1)])
+@pytest.mark.parametrize("M,N,K,splits", [(1, 1, 1, 1), (129, 63, 31, 1), (63, 131, 33, 1), (257, 67, 447, 2),
+                                          (2051, 4099, 37, 1)])
+def test_unaligned_edges(dev, M, N, K, ta, tb, splits):
+    """Tight odd rows (64x64_u, and 128x128_u for the last shape): every value
+    is loaded by itself and none past the last row's end (an odd M or N leaves
+    a pair's second row outside)."""
+    rng = np.random.default_rng(M + 3 * N + 7 * K + ta + 2 * tb)
+    A = rng.standard_normal((M, K)).astype(np.float32)
+    B = rng.standard_normal((K, N)).astype(np.float32)
+    As, Bs = [np.ascontiguousarray(x.T if t else x) for x, t in ((A, ta), (B, tb))]
+    dA, dB, dC = dev.upload(As), dev.upload(Bs), dev.upload(np.full((M, N), 7.0, np.float32))
+    try:
+        dev.force(None, splits)     # a forced split count leaves the 32x32 kernels out
+        dev.matmul(ta, tb, dA, dB, dC, M, N, K, As.shape[1], Bs.shape[1], N)
+        name = dev.last_variant()[0]
+        got = dev.download(dC, (M, N))
+    finally:
+        dev.force(None)
+        for p in (dA, dB, dC):
+            dev.free(p)
+    if As.shape[1] % 4 or Bs.shape[1] % 4:
+        assert name.endswith("_u")
+    want = A.astype(np.float64) @ B.astype(np.float64)
+    bound = (K + 8) * U * (np.abs(A).astype(np.float64) @ np.abs(B).astype(np.float64))
+    assert (np.abs(got - want) <= bound).all(), (name, float((np.abs(got - want) / np.maximum(bound, 1e-30)).max()))
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("tile", SPLIT_TILES)
 def test_row_sums_keep_no_common_error(dev, tile):
     """A of one sign against the same B: every row of C sums the same way, so a
@@ -136,19 +165,23 @@ def test_values_without_a_split(dev, tile, ta, tb):
 @pytest.mark.gpu
 @pytest.mark.parametrize("F,B,T", [(64, 2, 70), (320, 3, 129), (1024, 8, 1024)])
 def test_swiglu_epilogue_of_both_tiles(trlm, orc, F, B, T):
-    """The gate/up product with the SwiGLU epilogue, at sizes where the plan
-    takes the 64-wide and the 128-wide tile (the last), against the oracle's
-    logits."""
+    """The gate/up product with the SwiGLU epilogue, through the decoder's
+    prefill (whose engine takes the split products), at sizes where the plan
+    takes the 32-, the 64- and the 128-wide tile: the last position's logits
+    against the oracle's."""
     V, D, H, L = 150, 64, 2, 1
     model = orc.Model(V, D, H, L, F)
     params = model.init(1337, 1)
     ids = orc.random_tokens(B * T, V, 4242, 13, hi_exclusive=V)
     hm = trlm.HostModel(V, D, H, L, F, params)
-    tr = trlm.Trainer(hm, B, T)
+    tr = trlm.Trainer(hm, 1, 8)
+    dec = trlm.Decoder(tr, B, T + 1)
     try:
-        got = tr.forward_logits(ids)
+        dec.prefill(ids.reshape(B, T))
+        got = dec.logits()
     finally:
+        dec.destroy()
         tr.destroy()
         hm.close()
-    want = model.forward_logits(params, ids, B, T)
+    want = model.forward_logits(params, ids, B, T).reshape(B, T, V)[:, -1]
     assert np.abs(got - want).max() <= 1e-4 * np.abs(want).max()

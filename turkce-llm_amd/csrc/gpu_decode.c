@@ -43,6 +43,7 @@
 
 struct TrlmDecoder {
     GpuTrainer* g;
+    TrlmGemm* gemm;                     /* the prefill's products (made at the first prefill) */
     u32 B, ctx, len;
     u32 L, H, hd, D, F, V, ldv;
     f32 scale;
@@ -180,6 +181,7 @@ void gpu_decoder_destroy(TrlmDecoder* d) {
     hip_sync();
     drop_graph(d);
     free_prefill(d);
+    trlm_gemm_destroy(d->gemm);
     if (d->hist) hip_free(d->hist);
     if (d->u_all) hip_free(d->u_all);
     hip_free(d->pos_dev);
@@ -242,9 +244,11 @@ void gpu_decoder_prefill(TrlmDecoder* d, const u32* ids, u32 len) {
         d->pre_rows = R;
     }
     /* The trainer's forward on batch x len rows: a copy of the trainer with
-     * the same parameters, kernels and GEMM engine, whose activations are one
+     * the same parameters and kernels, whose activations are one
      * set of buffers shared by every layer (nothing is kept for a backward). */
     GpuTrainer pf = *g;
+    if (!d->gemm) d->gemm = trlm_gemm_create(&g->hip);   /* not the trainer's, which keeps to fp32 tiles */
+    pf.gemm = d->gemm;
     pf.B = d->B; pf.T = len; pf.N = (u32)R;
     for (u32 l = 0; l < g->L; l++) {
         GpuLayerActs* a = &pf.layers[l];

@@ -1,7 +1,4 @@
-// gemm.hip -- fp32 GEMMs on CDNA4 FP32 matrix cores (v_mfma_f32_32x32x2f32),
-// and the epilogues they share with gemm_split.hip.  The plan takes the
-// split-product kernels for aligned operands; the aligned variants here are
-// reached by trlm_gemm_force, the _u ones by operands without alignment.
+// gemm.hip -- fp32 GEMMs on CDNA4 FP32 matrix cores (v_mfma_f32_32x32x2f32).
 //
 // C[M,N] = alpha * op(A) @ op(B) (+ beta*C) (+ bias[n]) (+ resid[m,n])
 //   TA=0: A stored [M,K] (lda)     TA=1: A stored [K,M] -> op(A) = A^T
@@ -239,7 +236,10 @@ struct TileStream {
     static constexpr int NL = R * BK / 4 / 256;
     const float* ptr[NL];
     long long step;
-    __device__ __forceinline__ void init(const float* __restrict__ base, int ld, int r0, int rlim, int k0) {
+    // glu_F (m/n-major, R = 64): the tile's columns 0..31 are gate columns
+    // r0/2 .. of [gate | up] and 32..63 the matching up columns glu_F + r0/2 ..
+    __device__ __forceinline__ void init(const float* __restrict__ base, int ld, int r0, int rlim, int k0,
+                                         int glu_F = 0) {
         const int t = threadIdx.x;
 #pragma unroll
         for (int i = 0; i < NL; i++) {
@@ -248,6 +248,7 @@ struct TileStream {
             if (KMAJOR) { r = idx / (BK / 4); k = (idx % (BK / 4)) * 4; }
             else { k = idx / (R / 4); r = (idx % (R / 4)) * 4; }
             int gr = r0 + r;
+            if (!KMAJOR && glu_F) gr = (r < 32 ? 0 : glu_F - 32) + (r0 >> 1) + r;
             if (gr >= rlim) gr = KMAJOR ? rlim - 1 : 0;
             ptr[i] = KMAJOR ? base + (long long)gr * ld + (k0 + k) : base + (long long)(k0 + k) * ld + gr;
         }
@@ -815,7 +816,7 @@ __device__ __forceinline__ void gemm_epilogue(const GemmParams& p, float* C, con
 
 // SwiGLU epilogue of the gate/up projection (64x64 tiles, the B columns of
 // tile tn paired as gate r0/2 + 0..31 and up glu_F + r0/2 + 0..31, see
-// X3Tile): every wave stores its 32x32 block of C = [gate | up] (+ bias)
+// TileStream): every wave stores its 32x32 block of C = [gate | up] (+ bias)
 // at the real columns, the up waves hand their values to the gate waves
 // through LDS, and those store h = (g * sigmoid(g)) * u (feedforward.c:
 // 146-150, the order of k_swiglu_fwd) -- the separate SwiGLU pass and its
@@ -865,7 +866,106 @@ __device__ __forceinline__ void gemm_epilogue_glu(const GemmParams& p, const f32
     }
 }
 
-template <int TA, int TB, int BM, int BN, int BK, bool ALIGNED>
+// As gemm_mainloop_full, with the global loads two tiles ahead: tile j >= 1
+// is staged in register set (j - 1) & 1, so the load of tile kt + 3 is
+// issued at the end of tile kt and has two tiles of MFMAs to land before
+// its LDS store at the end of tile kt + 2.  The k loop is unrolled by two so
+// that the register set and the LDS buffer are compile-time indices.
+template <int TA, int TB, int BM, int BN, int BK, bool GLU = false>
+__device__ __forceinline__ void gemm_mainloop_pf2(const GemmParams& p, const float* A, const float* B, int m0,
+                                                  int n0, int kb, int ke, float* lds,
+                                                  f32x16 (&acc)[BM / 64][BN / 64], bool cs_on, f32x4& cs) {
+    constexpr bool AK = (TA == 0);
+    constexpr bool BK_ = (TB == 1);
+    constexpr int WM = BM / 2, WN = BN / 2;
+    constexpr int FM = WM / 32, FN = WN / 32;
+    constexpr int ASZ = TileLds<BM, BK, AK>::SIZE, BSZ = TileLds<BN, BK, BK_>::SIZE;
+    constexpr int NLA = BM * BK / 4 / 256, NLB = BN * BK / 4 / 256;
+    constexpr int NC = BK / 8;
+    static_assert(NC % 2 == 0, "fragment buffers alternate per 8-k chunk");
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int wm0 = (wave >> 1) * WM, wn0 = (wave & 1) * WN;
+
+    f32x4 ra[2][NLA], rb[2][NLB];
+    TileStream<BM, BK, AK> sa;
+    TileStream<BN, BK, BK_> sb;
+    sa.init(A, p.lda, m0, p.M, kb);
+    sb.init(B, p.ldb, n0, p.N, kb, GLU ? p.glu_F : 0);
+    const int nk = (ke - kb) / BK;
+    sa.load(ra[0]);
+    sb.load(rb[0]);
+    store_tile<BM, BK, AK>(lds, ra[0]);
+    store_tile<BN, BK, BK_>(lds + ASZ, rb[0]);
+    if (!BK_ && cs_on) colsum_add<BN, BK, NLB>(cs, rb[0]);
+    if (nk > 1) {
+        sa.load(ra[0]);
+        sb.load(rb[0]);
+    }
+    if (nk > 2) {
+        sa.load(ra[1]);
+        sb.load(rb[1]);
+    }
+    __syncthreads();
+    f32x4 fa[2][FM], fb[2][FN];
+    fetch_frags<BM, BK, AK, FM, GemmIlv<TA, TB, BM, BN, BK>::A>(lds, wm0, 0, lane, fa[0]);
+    fetch_frags<BN, BK, BK_, FN, GemmIlv<TA, TB, BM, BN, BK>::B>(lds + ASZ, wn0, 0, lane, fb[0]);
+    // one tile: kt is computed from LDS buffer S = kt & 1; tile kt + 1 sits in
+    // register set S and goes to buffer S ^ 1; set S then takes tile kt + 3
+    auto tile = [&](auto S_, int kt) {
+        constexpr int S = decltype(S_)::value;
+        const float* la = lds + S * (ASZ + BSZ);
+        float* ln = lds + (S ^ 1) * (ASZ + BSZ);
+#pragma unroll
+        for (int c = 0; c < NC; c++) {
+            const int u = c & 1, v = u ^ 1;
+            if (c + 1 < NC) {
+                fetch_frags<BM, BK, AK, FM, GemmIlv<TA, TB, BM, BN, BK>::A>(la, wm0, (c + 1) * 8, lane, fa[v]);
+                fetch_frags<BN, BK, BK_, FN, GemmIlv<TA, TB, BM, BN, BK>::B>(la + ASZ, wn0, (c + 1) * 8, lane, fb[v]);
+            } else {
+                if (kt + 1 < nk) {
+                    store_tile<BM, BK, AK>(ln, ra[S]);
+                    store_tile<BN, BK, BK_>(ln + ASZ, rb[S]);
+                    if (!BK_ && cs_on) colsum_add<BN, BK, NLB>(cs, rb[S]);
+                }
+                __syncthreads();
+                if (kt + 1 < nk) {
+                    fetch_frags<BM, BK, AK, FM, GemmIlv<TA, TB, BM, BN, BK>::A>(ln, wm0, 0, lane, fa[v]);
+                    fetch_frags<BN, BK, BK_, FN, GemmIlv<TA, TB, BM, BN, BK>::B>(ln + ASZ, wn0, 0, lane, fb[v]);
+                    if (kt + 3 < nk) {
+                        sa.load(ra[S]);
+                        sb.load(rb[S]);
+                    }
+                }
+            }
+#pragma unroll
+            for (int s = 0; s < 4; s++)
+#pragma unroll
+                for (int i = 0; i < FM; i++)
+#pragma unroll
+                    for (int j = 0; j < FN; j++)
+                        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(fb[u][j][s], fa[u][i][s], acc[i][j], 0, 0, 0);
+            // Spread this chunk's memory instructions between its MFMAs:
+            // groups of SG MFMAs (2 for the 16-MFMA chunks of 128x128, else
+            // 1), 1 LDS read, 1 global load, 1 LDS write (+2-4 % on the
+            // LM-head GEMMs against issuing them in one run beside a raised
+            // wave priority; the group size measured best per tile).
+            constexpr int SG = FM * FN >= 4 ? 2 : 1;
+#pragma unroll
+            for (int q = 0; q < 4 * FM * FN / SG; q++) {
+                __builtin_amdgcn_sched_group_barrier(0x008, SG, 0);  // MFMA
+                __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);   // LDS read
+                __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);   // global load
+                __builtin_amdgcn_sched_group_barrier(0x200, 1, 0);   // LDS write
+            }
+        }
+    };
+    for (int kt = 0; kt < nk; kt += 2) {
+        tile(std::integral_constant<int, 0>{}, kt);
+        if (kt + 1 < nk) tile(std::integral_constant<int, 1>{}, kt + 1);
+    }
+}
+
+template <int TA, int TB, int BM, int BN, int BK, bool ALIGNED, int PF = 1, bool GLU = false>
 __device__ __forceinline__ void gemm_body(const GemmParams& p) {
     constexpr bool AK = (TA == 0);   // A K-contiguous
     constexpr bool BK_ = (TB == 1);  // B K-contiguous
@@ -906,7 +1006,8 @@ __device__ __forceinline__ void gemm_body(const GemmParams& p) {
     f32x4 cs = {0.f, 0.f, 0.f, 0.f};
     if constexpr (ALIGNED) {
         if (kfull > kb) {
-            gemm_mainloop_full<TA, TB, BM, BN, BK>(p, A, B, m0, n0, kb, kfull, lds, acc, cs_on, cs);
+            if constexpr (PF == 2) gemm_mainloop_pf2<TA, TB, BM, BN, BK, GLU>(p, A, B, m0, n0, kb, kfull, lds, acc, cs_on, cs);
+            else gemm_mainloop_full<TA, TB, BM, BN, BK>(p, A, B, m0, n0, kb, kfull, lds, acc, cs_on, cs);
         }
         if (kfull < ke) {
             if (kfull > kb) __syncthreads();   // every wave is done reading the loop's LDS tiles
@@ -933,40 +1034,55 @@ __device__ __forceinline__ void gemm_body(const GemmParams& p) {
         }
     }
 
-    // the transposed store needs 32 rows of every wave's block in the operand LDS
-    constexpr bool LDS_STORE = 4 * 32 * (BN / 2) <= 2 * (ASZ + BSZ);
-    using Ilv = GemmIlv<TA, TB, BM, BN, BK>;
-    static_assert(Ilv::LDS_STORE == LDS_STORE, "one rule for the transposed store");
-    gemm_epilogue<BM, BN, LDS_STORE, Ilv::A, Ilv::B>(p, C, acc, m0 + wm0, n0 + wn0, lane,
-                                                     lds + wave * 32 * (BN / 2));
+    if constexpr (GLU) {
+        static_assert(BM == 64 && BN == 64 && PF == 2 && ALIGNED, "SwiGLU epilogue: 64x64 pipelined tiles");
+        gemm_epilogue_glu(p, acc[0][0], m0 + wm0, tn, wave >> 1, wave & 1, lane, lds);
+    } else {
+        // the transposed store needs 32 rows of every wave's block in the operand LDS
+        constexpr bool LDS_STORE = 4 * 32 * (BN / 2) <= 2 * (ASZ + BSZ);
+        using Ilv = GemmIlv<TA, TB, BM, BN, BK>;
+        static_assert(Ilv::LDS_STORE == LDS_STORE, "one rule for the transposed store");
+        gemm_epilogue<BM, BN, LDS_STORE, Ilv::A, Ilv::B>(p, C, acc, m0 + wm0, n0 + wn0, lane,
+                                                         lds + wave * 32 * (BN / 2));
+    }
 }
 
-#define GEMM_KERNEL(NAME, TA, TB, BM, BN, BK, AL, WPE)                                 \
+#define GEMM_KERNEL(NAME, TA, TB, BM, BN, BK, AL, WPE, PF)                             \
     extern "C" __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE))) \
     NAME(GemmParams p) {                                                                 \
-        gemm_body<TA, TB, BM, BN, BK, AL>(p);                                            \
+        gemm_body<TA, TB, BM, BN, BK, AL, PF>(p);                                        \
     }
 
-#define GEMM_LAYOUTS(TILE, BM, BN, BK, WPE)                                             \
-    GEMM_KERNEL(k_gemm_nn_##TILE, 0, 0, BM, BN, BK, true, WPE)                          \
-    GEMM_KERNEL(k_gemm_nt_##TILE, 0, 1, BM, BN, BK, true, WPE)                          \
-    GEMM_KERNEL(k_gemm_tn_##TILE, 1, 0, BM, BN, BK, true, WPE)
+#define GEMM_LAYOUTS(TILE, BM, BN, BK, WPE, PF)                                         \
+    GEMM_KERNEL(k_gemm_nn_##TILE, 0, 0, BM, BN, BK, true, WPE, PF)                      \
+    GEMM_KERNEL(k_gemm_nt_##TILE, 0, 1, BM, BN, BK, true, WPE, PF)                      \
+    GEMM_KERNEL(k_gemm_tn_##TILE, 1, 0, BM, BN, BK, true, WPE, PF)
 
 // name: k_gemm_<layout>_<BM>x<BN>[_k32][_u]
 //   _k32: 32-deep k step (one barrier per 32 k instead of 16)
 //   _u:   unaligned operands (scalar loads), 16-deep k step
 // Waves own (BM/2)x(BN/2).  WPE is the register budget as resident waves per
 // SIMD: the largest count the variant's LDS allows (2 for the
-// 8-accumulator-block 256x128 / 128x256 tiles), short of spilling.
-GEMM_LAYOUTS(256x128, 256, 128, 16, 2)
-GEMM_LAYOUTS(128x256, 128, 256, 16, 2)
-GEMM_LAYOUTS(128x128_k32, 128, 128, 32, 2)
-GEMM_LAYOUTS(64x128, 64, 128, 16, 4)
-GEMM_LAYOUTS(64x64, 64, 64, 16, 5)
-GEMM_KERNEL(k_gemm_nn_64x64_u, 0, 0, 64, 64, 16, false, 1)
-GEMM_KERNEL(k_gemm_nt_64x64_u, 0, 1, 64, 64, 16, false, 1)
-GEMM_KERNEL(k_gemm_tn_64x64_u, 1, 0, 64, 64, 16, false, 1)
-GEMM_KERNEL(k_gemm_tt_64x64_u, 1, 1, 64, 64, 16, false, 1)
+// 8-accumulator-block 256x128 / 128x256 tiles), short of spilling.  PF is the
+// interior loop's global-load distance in tiles (2 where the second staging
+// register set fits the budget: 2-5 % faster on the model's shapes).
+GEMM_LAYOUTS(256x128, 256, 128, 16, 2, 1)
+GEMM_LAYOUTS(128x256, 128, 256, 16, 2, 1)
+GEMM_LAYOUTS(128x128, 128, 128, 16, 3, 2)
+GEMM_LAYOUTS(128x128_k32, 128, 128, 32, 2, 1)
+GEMM_LAYOUTS(64x128, 64, 128, 16, 4, 1)
+GEMM_LAYOUTS(64x128_k32, 64, 128, 32, 2, 2)
+GEMM_LAYOUTS(64x64, 64, 64, 16, 5, 1)
+GEMM_LAYOUTS(64x64_k32, 64, 64, 32, 4, 2)
+// the gate/up projection with the SwiGLU epilogue (host: K % 32 == 0, N = 2F, F % 32 == 0)
+extern "C" __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4)))
+k_gemm_nn_64x64_k32_glu(GemmParams p) {
+    gemm_body<0, 0, 64, 64, 32, true, 2, true>(p);
+}
+GEMM_KERNEL(k_gemm_nn_64x64_u, 0, 0, 64, 64, 16, false, 1, 1)
+GEMM_KERNEL(k_gemm_nt_64x64_u, 0, 1, 64, 64, 16, false, 1, 1)
+GEMM_KERNEL(k_gemm_tn_64x64_u, 1, 0, 64, 64, 16, false, 1, 1)
+GEMM_KERNEL(k_gemm_tt_64x64_u, 1, 1, 64, 64, 16, false, 1, 1)
 
 // out[m,n] = alpha * sum_s W[s][m,n] (+ beta*out) (+ bias[n]); out = resid + v.
 // Partials are summed in split order, so the result is reproducible.

@@ -62,7 +62,9 @@ constexpr int X3_FLIP = 4;    // steps between changes of the sum's sign
 // One operand's part of a k step: R rows (of m or n) by 32 k.
 // LDS: [plane h/m/l][chunk c of 8 k][slot], 16 bytes each; chunk c holds
 // k = 4c..4c+3 and 16+4c..16+4c+3 (the same for both operands).
-template <int R, bool KM>
+// AL: rows 16-byte aligned (ld a multiple of 4), so that four k or two rows are one
+// load; without it every value is loaded by itself.
+template <int R, bool KM, bool AL>
 struct X3Tile {
     static constexpr int W = (!KM && R >= 128) ? 2 : 1;     // rows per thread and id
     static constexpr int NI = R * 4 / 256 / W;              // ids per thread
@@ -71,6 +73,7 @@ struct X3Tile {
     static constexpr bool ILV = W == 2;
     float x[NI * W][8];
     const float* ptr[NI];
+    int second[NI];          // unaligned: the second row's offset (0 where it would be past the edge)
     long long step, ld;
 
     __device__ __forceinline__ static int slot(int r) { return ILV ? (r & ~63) + ((r & 63) >> 1) + 32 * (r & 1) : r; }
@@ -89,6 +92,7 @@ struct X3Tile {
                 int gr = r0 + r;
                 if (glu_F) gr = (r < R / 2 ? 0 : glu_F - R / 2) + (r0 >> 1) + r;
                 if (gr >= rlim) gr = 0;
+                second[i] = AL || gr + 1 < rlim;
                 ptr[i] = base + (long long)(k0 + 4 * (id / (R / W))) * ld + gr;
             }
         }
@@ -100,7 +104,10 @@ struct X3Tile {
         for (int i = 0; i < NI; i++) {
 #pragma unroll
             for (int j = 0; j < 2; j++) {
-                if constexpr (KM) {
+                if constexpr (KM && !AL) {
+#pragma unroll
+                    for (int e = 0; e < 4; e++) x[i][4 * j + e] = ptr[i][16 * j + e];
+                } else if constexpr (KM) {
                     const f32x4 v = *(const f32x4*)(ptr[i] + 16 * j);
 #pragma unroll
                     for (int e = 0; e < 4; e++) x[i][4 * j + e] = v[e];
@@ -108,7 +115,10 @@ struct X3Tile {
 #pragma unroll
                     for (int e = 0; e < 4; e++) {
                         const float* src = ptr[i] + (16 * j + e) * ld;
-                        if constexpr (W == 2) {
+                        if constexpr (W == 2 && !AL) {
+                            x[2 * i][4 * j + e] = src[0];
+                            x[2 * i + 1][4 * j + e] = src[second[i]];
+                        } else if constexpr (W == 2) {
                             const f32x2 v = *(const f32x2*)src;
                             x[2 * i][4 * j + e] = v[0];
                             x[2 * i + 1][4 * j + e] = v[1];
@@ -135,7 +145,7 @@ struct X3Tile {
                 const bool in = k0 + kk < rem;
 #pragma unroll
                 for (int w = 0; w < W; w++)
-                    x[W * i + w][j] = in ? (KM ? src[kk] : src[kk * ld + w]) : 0.f;
+                    x[W * i + w][j] = in ? (KM ? src[kk] : src[kk * ld + (w ? second[i] : 0)]) : 0.f;
             }
         }
     }
@@ -264,11 +274,11 @@ __device__ __forceinline__ void gemm_wave_f32(const GemmParams& p, const float* 
     }
 }
 
-template <int TA, int TB, int BM, int BN, bool GLU = false>
+template <int TA, int TB, int BM, int BN, bool AL = true, bool GLU = false>
 __device__ __forceinline__ void gemm_x3_body(const GemmParams& p) {
     constexpr int FM = BM / 64, FN = BN / 64;
-    using TileA = X3Tile<BM, TA == 0>;
-    using TileB = X3Tile<BN, TB == 1>;
+    using TileA = X3Tile<BM, TA == 0, AL>;
+    using TileB = X3Tile<BN, TB == 1, AL>;
     __shared__ u32x4 lds[TileA::UNITS + TileB::UNITS];
     u32x4* la = lds;
     u32x4* lb = lds + TileA::UNITS;
@@ -430,17 +440,30 @@ __device__ __forceinline__ void gemm_x3_body(const GemmParams& p) {
         gemm_x3_body<TA, TB, BM, BN>(p);                                                           \
     }
 #define GEMM_X3_LAYOUTS(TILE, BM, BN, WPE)              \
-    GEMM_X3(k_gemm_nn_##TILE, 0, 0, BM, BN, WPE)        \
-    GEMM_X3(k_gemm_nt_##TILE, 0, 1, BM, BN, WPE)        \
-    GEMM_X3(k_gemm_tn_##TILE, 1, 0, BM, BN, WPE)
+    GEMM_X3(k_xgemm_nn_##TILE, 0, 0, BM, BN, WPE)        \
+    GEMM_X3(k_xgemm_nt_##TILE, 0, 1, BM, BN, WPE)        \
+    GEMM_X3(k_xgemm_tn_##TILE, 1, 0, BM, BN, WPE)
 GEMM_X3_LAYOUTS(128x128, 128, 128, 3)
 GEMM_X3_LAYOUTS(64x128_k32, 64, 128, 4)
 GEMM_X3_LAYOUTS(64x64_k32, 64, 64, 5)
+// unaligned operands
+#define GEMM_X3_U(NAME, TA, TB, BM, BN, WPE)                                                      \
+    extern "C" __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE)))   \
+    NAME(GemmParams p) {                                                                           \
+        gemm_x3_body<TA, TB, BM, BN, false>(p);                                                    \
+    }
+GEMM_X3_U(k_xgemm_nn_64x64_u, 0, 0, 64, 64, 5)
+GEMM_X3_U(k_xgemm_nt_64x64_u, 0, 1, 64, 64, 5)
+GEMM_X3_U(k_xgemm_tn_64x64_u, 1, 0, 64, 64, 5)
+GEMM_X3_U(k_xgemm_tt_64x64_u, 1, 1, 64, 64, 5)
+GEMM_X3_U(k_xgemm_nn_128x128_u, 0, 0, 128, 128, 3)
+GEMM_X3_U(k_xgemm_nt_128x128_u, 0, 1, 128, 128, 3)
+GEMM_X3_U(k_xgemm_tn_128x128_u, 1, 0, 128, 128, 3)
 // the gate/up projection with the SwiGLU epilogue (host: K % 32 == 0, N = 2F, F a multiple of half the tile)
 #define GEMM_X3_GLU(NAME, BM, BN, WPE)                                                            \
     extern "C" __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE)))   \
     NAME(GemmParams p) {                                                                           \
-        gemm_x3_body<0, 0, BM, BN, true>(p);                                                       \
+        gemm_x3_body<0, 0, BM, BN, true, true>(p);                                                       \
     }
-GEMM_X3_GLU(k_gemm_nn_64x64_k32_glu, 64, 64, 5)
-GEMM_X3_GLU(k_swiglu_gemm_128x128, 128, 128, 3)
+GEMM_X3_GLU(k_xgemm_nn_64x64_k32_glu, 64, 64, 5)
+GEMM_X3_GLU(k_xgemm_nn_128x128_glu, 128, 128, 3)

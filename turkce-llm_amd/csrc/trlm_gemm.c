@@ -13,7 +13,7 @@
  *     that k_gemm_splitk_reduce sums in split order, so the result stays
  *     deterministic (no atomics);
  *   - operands whose rows are not 16-byte aligned go to the _u variants,
- *     which use scalar loads.
+ *     which load value by value.
  */
 #include <stdint.h>
 #include <stdio.h>
@@ -28,30 +28,36 @@
 enum { L_NN = 0, L_NT = 1, L_TN = 2 };
 static const char* LAYOUT_NAME[4] = { "nn", "nt", "tn", "tt" };
 
-/* Aligned tile variants: name suffix, tile rows/cols, k step.  128x128,
- * 64x128_k32 and 64x64_k32 form their products on the bf16 matrix cores from
- * exact three-way splits (gemm_split.hip); the others, which only
- * trlm_gemm_force selects, use the fp32 matrix cores (gemm.hip). */
+/* Aligned tile variants: name suffix, tile rows/cols, k step of the fp32
+ * kernels (gemm.hip).  128x128, 64x128_k32 and 64x64_k32 also come from exact
+ * three-way bf16 splits (gemm_split.hip, k step 32), which an engine takes
+ * for them unless it keeps to fp32. */
 typedef struct TileDef { const char* name; int bm, bn, bk; } TileDef;
 enum { T_256x128, T_128x256, T_128x128, T_128x128_K32, T_64x128, T_64x128_K32, T_64x64, T_64x64_K32, T_COUNT };
 static const TileDef TILES[T_COUNT] = {
-    { "256x128", 256, 128, 16 }, { "128x256", 128, 256, 16 }, { "128x128", 128, 128, 32 },
+    { "256x128", 256, 128, 16 }, { "128x256", 128, 256, 16 }, { "128x128", 128, 128, 16 },
     { "128x128_k32", 128, 128, 32 }, { "64x128", 64, 128, 16 }, { "64x128_k32", 64, 128, 32 },
     { "64x64", 64, 64, 16 }, { "64x64_k32", 64, 64, 32 },
 };
+
+static int has_split(int t) { return t == T_128x128 || t == T_64x128_K32 || t == T_64x64_K32; }
 
 #define CUS 256
 #define KCHUNK_ALIGN 32  /* split-K chunks are multiples of every variant's k step */
 
 struct TrlmGemm {
     HipCtx* ctx;
-    hipFunction_t k[3][T_COUNT];
-    hipFunction_t ku[4];
+    hipFunction_t k[3][T_COUNT];   /* fp32 tiles (gemm.hip) */
+    hipFunction_t x[3][T_COUNT];   /* split products (gemm_split.hip), for the tiles that have them */
+    int fp32;                      /* keep to the fp32 tiles */
+    hipFunction_t ku[4];           /* unaligned operands: fp32 64x64_u */
+    hipFunction_t xu[4], xu128[3]; /* the same from split products, 64x64_u and 128x128_u */
     hipFunction_t reduce;
     hipFunction_t reduce4;   /* four columns per thread, for 16-byte aligned operands */
     hipFunction_t small[2][3];   /* k_smallgemm_<layout>[_u]: 32x32 tiles, k shared out over a workgroup's waves */
     hipFunction_t small_glu;
-    hipFunction_t glu, glu128;   /* SwiGLU epilogue: k_gemm_nn_64x64_k32_glu, k_swiglu_gemm_128x128 */
+    hipFunction_t glu;             /* SwiGLU epilogue: fp32 64x64_k32 */
+    hipFunction_t xglu, xglu128;   /* split products, 64x64_k32 and 128x128 */
     hipDeviceptr_t ws;
     u64 ws_floats;
     char last[48];
@@ -69,10 +75,18 @@ TrlmGemm* trlm_gemm_create(HipCtx* ctx) {
         for (int t = 0; t < T_COUNT; t++) {
             snprintf(name, sizeof(name), "k_gemm_%s_%s", LAYOUT_NAME[l], TILES[t].name);
             e->k[l][t] = hip_get_kernel(ctx, name);
+            if (!has_split(t)) continue;
+            snprintf(name, sizeof(name), "k_xgemm_%s_%s", LAYOUT_NAME[l], TILES[t].name);
+            e->x[l][t] = hip_get_kernel(ctx, name);
         }
     for (int l = 0; l < 4; l++) {
         snprintf(name, sizeof(name), "k_gemm_%s_64x64_u", LAYOUT_NAME[l]);
         e->ku[l] = hip_get_kernel(ctx, name);
+        snprintf(name, sizeof(name), "k_xgemm_%s_64x64_u", LAYOUT_NAME[l]);
+        e->xu[l] = hip_get_kernel(ctx, name);
+        if (l == 3) break;
+        snprintf(name, sizeof(name), "k_xgemm_%s_128x128_u", LAYOUT_NAME[l]);
+        e->xu128[l] = hip_get_kernel(ctx, name);
     }
     for (int l = 0; l < 3; l++)
         for (int u = 0; u < 2; u++) {
@@ -84,10 +98,19 @@ TrlmGemm* trlm_gemm_create(HipCtx* ctx) {
     e->reduce = hip_get_kernel(ctx, "k_gemm_splitk_reduce");
     e->reduce4 = hip_get_kernel(ctx, "k_gemm_splitk_reduce4");
     e->glu = hip_get_kernel(ctx, "k_gemm_nn_64x64_k32_glu");
-    e->glu128 = hip_get_kernel(ctx, "k_swiglu_gemm_128x128");
+    e->xglu = hip_get_kernel(ctx, "k_xgemm_nn_64x64_k32_glu");
+    e->xglu128 = hip_get_kernel(ctx, "k_xgemm_nn_128x128_glu");
     trlm_noalloc_setup(ctx->device);
     return e;
 }
+
+/* The engine's products keep to the fp32 matrix cores, with the tiles and
+ * split-K of the fp32 plan.  The trainer's engines do: a training run's bits
+ * are those of the fp32 tiles, and an optimizer's first steps magnify any
+ * other rounding, however small (AdamW divides by the gradient's size: after
+ * one step of the 12-layer model two correct roundings of it, each 1.7e-6 or
+ * less from 64 bits, have gradients 7e-6 to 2e-5 apart). */
+void trlm_gemm_keep_fp32(TrlmGemm* e) { e->fp32 = 1; }
 
 void trlm_gemm_destroy(TrlmGemm* e) {
     if (!e) return;
@@ -233,6 +256,80 @@ static void select_plan(int M, int N, int K, u32 batch, int* tile, int* splits) 
         }
 }
 
+/* Plan model of the fp32 tiles (an engine that keeps them, see
+ * trlm_gemm_keep_fp32): the tiles' workgroups are spread evenly over the 256 CUs, so
+ * the busiest CU runs n = ceil(workgroups / 256) of them, `occ` at a time
+ * (the variant's resident workgroups per CU).  A CU with c resident
+ * workgroups runs at fp32_cu_rate(c) of its steady-state rate (one resident
+ * 4-wave workgroup cannot hide its own load latency), and each variant has
+ * its own steady-state efficiency.  The last resident batch adds an
+ * imbalance term proportional to a workgroup's duration.  Split-K adds the
+ * partials' round trip through HBM plus the reduction launch.  Constants
+ * fitted to MI355X timings of every variant/split on the model's GEMMs at
+ * 512-8192 rows (within 0.6 % of the per-shape best over those 45 shapes). */
+typedef struct Fp32Tile { int tile; int occ; double eff; } Fp32Tile;
+static const Fp32Tile FP32_TILES[] = {
+    { T_128x128, 3, 1.047 }, { T_128x256, 2, 0.977 }, { T_256x128, 2, 1.008 },
+    { T_64x128_K32, 2, 0.955 }, { T_64x64_K32, 4, 0.992 },
+};
+#define FP32_CU_FLOPS 0.6e12     /* per-CU steady-state fp32 MFMA rate, FLOP/s */
+#define FP32_SPLIT_BW 1.63e12    /* effective bytes/s of the partials' round trip */
+#define FP32_SPLIT_FIXED 1.25e-6 /* reduction launch, s */
+#define FP32_TAIL 0.075          /* last-round imbalance, in resident-batch durations */
+
+static double fp32_cu_rate(int c) { return c <= 1 ? 0.916 : 1.0; }
+
+static double fp32_cost(const Fp32Tile* pt, int M, int N, int K, u32 batch, int splits) {
+    const TileDef* td = &TILES[pt->tile];
+    double wg = (double)cdiv(M, td->bm) * cdiv(N, td->bn) * batch * splits;
+    int kch = splits > 1 ? cdiv(cdiv(K, splits), KCHUNK_ALIGN) * KCHUNK_ALIGN : K;
+    long long n = (long long)((wg + CUS - 1) / CUS);
+    double w = 2.0 * td->bm * td->bn * (double)kch / (pt->eff * FP32_CU_FLOPS);
+    long long full = n / pt->occ, rest = n % pt->occ;
+    double t = (double)full * pt->occ * w / fp32_cu_rate(pt->occ);
+    if (rest) t += (double)rest * w / fp32_cu_rate((int)rest);
+    /* workgroups of one resident batch finish unevenly: long workgroups
+     * leave CUs idle at the end, which more, shorter ones even out */
+    t += FP32_TAIL * pt->occ * w / fp32_cu_rate((int)(n < pt->occ ? n : pt->occ));
+    if (splits > 1) t += (splits + 1) * (double)M * N * 4.0 / FP32_SPLIT_BW + FP32_SPLIT_FIXED;
+    return t;
+}
+
+static void select_fp32(int M, int N, int K, u32 batch, int* tile, int* splits) {
+    double best = 0.0;
+    *tile = T_128x128;
+    *splits = 1;
+    /* Decode-sized products (M <= 128 rows, few tiles): each workgroup's
+     * k loop is latency-bound (~1 us per 32-deep step), so split K down to
+     * 64-deep chunks over up to 8 partitions, one workgroup per CU at most.
+     * Measured on MI355X at M = 64: QKV 12.8 -> 9.0 us, attention-out 11.8
+     * -> 8.6, gate_up 12.4 -> 8.2, down (K = 1024) 12.6 -> 10.4, reduction
+     * included. */
+    if (M <= 128 && batch == 1) {
+        long long tiles = (long long)cdiv(M, 64) * cdiv(N, 64);
+        if (tiles < 128) {
+            long long smax = K / 64;
+            if (smax > 8) smax = 8;
+            if (smax > CUS / tiles) smax = CUS / tiles;
+            *tile = T_64x64_K32;
+            for (size_t j = 0; j < sizeof(PLAN_SPLITS) / sizeof(PLAN_SPLITS[0]); j++)
+                if (PLAN_SPLITS[j] <= smax) *splits = PLAN_SPLITS[j];
+            return;
+        }
+    }
+    for (size_t i = 0; i < sizeof(FP32_TILES) / sizeof(FP32_TILES[0]); i++)
+        for (size_t j = 0; j < sizeof(PLAN_SPLITS) / sizeof(PLAN_SPLITS[0]); j++) {
+            int sp = PLAN_SPLITS[j];
+            if (sp > 1 && (batch != 1 || K / sp < 256)) continue;
+            double c = fp32_cost(&FP32_TILES[i], M, N, K, batch, sp);
+            if ((i == 0 && j == 0) || c < best) {
+                best = c;
+                *tile = FP32_TILES[i].tile;
+                *splits = sp;
+            }
+        }
+}
+
 /* Products of few tiles (gemm_small.hip, reported as the tile 32x32): one
  * 32x32 tile per workgroup, k shared out over its waves.  Up to two tiles per
  * CU, measured on MI355X against the planned tile (us): 64x1152x384 5.8 / 8.0,
@@ -241,12 +338,12 @@ static void select_plan(int M, int N, int K, u32 batch, int* tile, int* splits) 
  * than 96 k up to one tile per CU (384x1152x64, 432 tiles: 5.2 / 4.9).  Up to
  * 768 k, 1152 where neither side is at most 128 (512x384x1024 11.0 / 13.4,
  * 358x137x1099 12.9 / 14.6, but 64x384x1024, which select_plan splits into
- * more partitions, 10.8 / 9.4).  Unaligned operands, whose other kernel has no
- * split: up to four tiles per CU (1000x701x333 16.3 / 19.8, but 2001x1001x333
- * 34.8 / 30.1). */
+ * more partitions, 10.8 / 9.4).  Unaligned operands, which this kernel loads
+ * with the fewer idle lanes, up to three tiles per CU where k is short (704
+ * tiles: 701x1001x101 7.3 / 9.2, but 1000x701x333 17.2 / 14.9). */
 static int small_gemm(int M, int N, int K, u32 batch, int aligned) {
     const long long tiles = (long long)cdiv(M, 32) * cdiv(N, 32);
-    const int most = !aligned ? 4 * CUS : K >= 96 ? 2 * CUS : CUS;
+    const int most = !aligned && K <= 192 ? 3 * CUS : K >= 96 ? 2 * CUS : CUS;
     return batch == 1 && K <= (M > 128 && N > 128 ? 1152 : 768) && tiles <= most;
 }
 
@@ -324,22 +421,14 @@ i32 trlm_gemm_ws(TrlmGemm* e, i32 trans_a, i32 trans_b, hipDeviceptr_t A, hipDev
         p.splits = 1; p.kchunk = K; p.alpha = alpha; p.beta = 0.0f;
         /* the 128-wide tile where F holds whole half tiles and the plan
          * model finds it the faster of the two */
-        if (small_gemm(M, N, K, 1, 1)) {
-            p.tiles_m = cdiv(M, 32); p.tiles_n = N / 32;
-            p.glu_h = (float*)x->glu_h; p.glu_F = x->glu_F;
-            snprintf(e->last, sizeof(e->last), "k_gemm_%s_32x32_glu", LAYOUT_NAME[L_NN]);
-            e->last_splits = small_splits(K);
-            launch(e->small_glu, &p, 1);
-            return 0;
-        }
-        const int wide = x->glu_F % 64 == 0 && plan_cost(&PLAN_TILES[0], M, N, K, 1, 1) <
-                                                   plan_cost(&PLAN_TILES[2], M, N, K, 1, 1);
+        const int wide = !e->fp32 && x->glu_F % 64 == 0 && plan_cost(&PLAN_TILES[0], M, N, K, 1, 1) <
+                                                               plan_cost(&PLAN_TILES[2], M, N, K, 1, 1);
         const int tile = wide ? 128 : 64;
         p.tiles_m = cdiv(M, tile); p.tiles_n = cdiv(N, tile);
         p.glu_h = (float*)x->glu_h; p.glu_F = x->glu_F;
-        snprintf(e->last, sizeof(e->last), wide ? "k_swiglu_gemm_128x128" : "k_gemm_nn_64x64_k32_glu");
+        snprintf(e->last, sizeof(e->last), "k_gemm_%s_%s_glu", LAYOUT_NAME[L_NN], wide ? "128x128" : "64x64_k32");
         e->last_splits = 1;
-        launch(wide ? e->glu128 : e->glu, &p, 1);
+        launch(e->fp32 ? e->glu : wide ? e->xglu128 : e->xglu, &p, 1);
         return 0;
     }
     if (csum && (batch != 1 || trans_b)) {
@@ -380,23 +469,23 @@ i32 trlm_gemm_ws(TrlmGemm* e, i32 trans_a, i32 trans_b, hipDeviceptr_t A, hipDev
         launch(e->small[!aligned][layout], &p, 1);
         return 0;
     }
-    if (!aligned) {
-        p.tiles_m = cdiv(M, 64); p.tiles_n = cdiv(N, 64);
-        snprintf(e->last, sizeof(e->last), "k_gemm_%s_64x64_u", LAYOUT_NAME[layout]);
-        e->last_splits = 1;
-        if (stats) set_stats(&p, stats, stats_cap, 64);
-        launch(e->ku[layout], &p, batch);
-        return p.stats ? 2 * p.tiles_n : 0;
-    }
-
     int tile, splits;
-    select_plan(M, N, K, batch, &tile, &splits);
-    if (e->force_tile >= 0) {
+    if (e->fp32) select_fp32(M, N, K, batch, &tile, &splits);
+    else select_plan(M, N, K, batch, &tile, &splits);
+    if (!aligned) {
+        /* the unaligned kernels: one fp32 tile without split-K, two of the
+         * split products' tiles */
+        if (e->fp32 || tile != T_128x128 || layout == 3 || stats) tile = T_64x64_K32;
+        if (e->fp32 || layout == 3) splits = 1;
+    } else if (e->force_tile >= 0) {
         tile = e->force_tile;
         splits = batch == 1 ? auto_splits(tiles_of(tile, M, N, 1), K) : 1;
     }
-    if (e->force_splits > 0 && batch == 1) splits = e->force_splits;
+    if (e->force_splits > 0 && batch == 1 && (aligned || (!e->fp32 && layout != 3))) splits = e->force_splits;
     if (stats || rope) splits = 1;         /* these epilogues need whole sums */
+    hipFunction_t kernel = e->k[layout < 3 ? layout : 0][tile];
+    if (!aligned) kernel = e->fp32 ? e->ku[layout] : tile == T_128x128 ? e->xu128[layout] : e->xu[layout];
+    else if (!e->fp32 && has_split(tile)) kernel = e->x[layout][tile];
     p.tiles_m = cdiv(M, TILES[tile].bm);
     p.tiles_n = cdiv(N, TILES[tile].bn);
     if (stats) set_stats(&p, stats, stats_cap, TILES[tile].bn);
@@ -422,10 +511,11 @@ i32 trlm_gemm_ws(TrlmGemm* e, i32 trans_a, i32 trans_b, hipDeviceptr_t A, hipDev
             splits = cdiv(K, kchunk);
         }
     }
-    snprintf(e->last, sizeof(e->last), "k_gemm_%s_%s", LAYOUT_NAME[layout], TILES[tile].name);
+    snprintf(e->last, sizeof(e->last), "k_gemm_%s_%s", LAYOUT_NAME[layout],
+             aligned ? TILES[tile].name : tile == T_128x128 ? "128x128_u" : "64x64_u");
     e->last_splits = splits;
     if (splits <= 1) {
-        launch(e->k[layout][tile], &p, batch);
+        launch(kernel, &p, batch);
         return p.stats ? 2 * p.tiles_n : 0;
     }
     u64 need = (u64)splits * slab;
@@ -445,7 +535,7 @@ i32 trlm_gemm_ws(TrlmGemm* e, i32 trans_a, i32 trans_b, hipDeviceptr_t A, hipDev
     q.kchunk = kchunk;
     q.splits = splits;
     q.alpha = 1.0f; q.beta = 0.0f; q.bias = NULL; q.resid = NULL;
-    launch(e->k[layout][tile], &q, (u32)splits);
+    launch(kernel, &q, (u32)splits);
     long long total = (long long)slab;
     i32 sp = splits;
     i64 sW = (i64)slab;
