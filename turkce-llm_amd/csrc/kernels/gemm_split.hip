@@ -11,10 +11,13 @@
 // rounded is the running sum, as with the fp32 matrix cores, and less often
 // (6 times per 16 k instead of 8).  Error against 64 bits, N(0,1) x
 // N(0,0.02): K = 384 2.9e-7 (fp32 MFMA 3.5e-7), K = 8192 in one sum 1.4e-6
-// (1.6e-6); a training step's gradients 1.1e-6 (1.7e-6).
+// (1.6e-6).
 //
-// Why: the fp32 matrix cores (157 TFLOP/s) were 79-86 % busy, so the GEMMs,
-// 70 % of a training step, could only gain from another unit.  Six bf16
+// Serves raw GEMMs, the matmul node and the decoder's prefill; the trainer
+// keeps the fp32 tiles (trlm_gemm_keep_fp32), whose rounding its results pin.
+//
+// Why: the fp32 matrix cores (157 TFLOP/s) were 79-86 % busy, so large GEMMs
+// could only gain from another unit.  Six bf16
 // products at the 2.0 PFLOP/s that the matrix cores sustain on random data
 // are worth 333 TFLOP/s.  Measured before -> after: LM head forward
 // 8192x31769x384 1526 -> 1050 us, gate/up 8192x2048x384 105 -> 75 us,
