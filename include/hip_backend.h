@@ -56,6 +56,9 @@ hipDeviceptr_t hip_alloc(u64 bytes);                          /* cuda_backend.h:
 void hip_free(hipDeviceptr_t p);
 void hip_h2d(hipDeviceptr_t dst, const void* src, u64 bytes);
 void hip_d2h(void* dst, hipDeviceptr_t src, u64 bytes);
+/* Not in the reference's backend: hip_d2h of `rows` rows of row_bytes, stored
+ * `pitch` bytes apart (pitch >= row_bytes), to packed rows at dst. */
+void hip_d2h_rows(void* dst, hipDeviceptr_t src, u64 pitch, u64 row_bytes, u64 rows);
 
 void hip_launch_1d(hipFunction_t f, u32 n, void** params);    /* cuda_backend.h:50-60 */
 void hip_launch_2d(hipFunction_t f, u32 rows, u32 cols, void** params);

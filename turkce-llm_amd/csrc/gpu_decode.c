@@ -405,8 +405,7 @@ void gpu_decoder_step(TrlmDecoder* d, const u32* ids) {
 
 void gpu_decoder_logits(TrlmDecoder* d, f32* host_logits) {
     trlm_bind(d->g);
-    for (u32 b = 0; b < d->B; b++)
-        hip_d2h(host_logits + (u64)b * d->V, at(d->logits, (u64)b * d->ldv), (u64)d->V * F4);
+    hip_d2h_rows(host_logits, d->logits, (u64)d->ldv * F4, (u64)d->V * F4, d->B);
 }
 
 void gpu_decoder_greedy(TrlmDecoder* d, u32* out_ids) {

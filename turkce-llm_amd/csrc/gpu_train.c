@@ -872,9 +872,7 @@ void trlm_eval_queued(GpuTrainer* g, hipDeviceptr_t sum, i32 acc) {
 /* ---------------- additive entry points (trlm_ext.h) ---------------- */
 
 static void logits_to_host(GpuTrainer* g, f32* host) {
-    hipError_t r = hipMemcpy2DAsync(host, (size_t)g->V * F4, g->logits, (size_t)g->ldv * F4, (size_t)g->V * F4,
-                                    g->N, hipMemcpyDeviceToHost, g->hip.stream);
-    if (r != hipSuccess) fatal("logits copy failed");
+    hip_d2h_rows(host, g->logits, (u64)g->ldv * F4, (u64)g->V * F4, g->N);
     hip_sync();
 }
 
