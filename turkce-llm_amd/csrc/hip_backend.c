@@ -275,7 +275,7 @@ static void copy_rows(u8* dst, const u8* src, u64 pitch, u64 row_bytes, u64 rows
 
 void hip_h2d(hipDeviceptr_t dst, const void* src, u64 bytes) {
     HipCtx* c = current("hip_h2d");
-    const int staged = bytes > 0 && bytes <= STAGED_SMALL;
+    const int staged = src && bytes > 0 && bytes <= STAGED_SMALL;   /* no host address: the runtime's error */
     if (staged) {
         u8* stage = stage_acquire(c)[0];
         memcpy(stage, src, bytes);
@@ -307,7 +307,7 @@ static void d2h_blocks(HipCtx* c, u8* dst, const u8* src, u64 pitch, u64 row_byt
 
 void hip_d2h(void* dst, hipDeviceptr_t src, u64 bytes) {
     HipCtx* c = current("hip_d2h");
-    if (bytes > STAGED_SMALL && bytes < COPY_THREADED) {
+    if (!dst || (bytes > STAGED_SMALL && bytes < COPY_THREADED)) {
         check(hipMemcpyDtoHAsync(dst, src, bytes, c->stream), "hipMemcpyDtoHAsync");
         check(hipStreamSynchronize(c->stream), "hipStreamSynchronize");
         return;
@@ -319,13 +319,13 @@ void hip_d2h(void* dst, hipDeviceptr_t src, u64 bytes) {
 
 void hip_d2h_rows(void* dst, hipDeviceptr_t src, u64 pitch, u64 row_bytes, u64 rows) {
     HipCtx* c = current("hip_d2h_rows");
-    if (pitch <= STAGE_BLOCK && pitch > row_bytes && row_bytes > 0) {
+    if (dst && pitch <= STAGE_BLOCK && pitch > row_bytes && row_bytes > 0) {
         d2h_blocks(c, (u8*)dst, (const u8*)src, pitch, row_bytes, rows, STAGE_BLOCK / pitch);
     } else if (pitch == row_bytes) {
         hip_d2h(dst, src, rows * row_bytes);
     } else {
         for (u64 r = 0; r < rows; r++)
-            hip_d2h((u8*)dst + r * row_bytes, (hipDeviceptr_t)((u8*)src + r * pitch), row_bytes);
+            hip_d2h(dst ? (u8*)dst + r * row_bytes : NULL, (hipDeviceptr_t)((u8*)src + r * pitch), row_bytes);
     }
 }
 
