@@ -185,3 +185,31 @@ def test_swiglu_epilogue_of_both_tiles(trlm, orc, F, B, T):
         hm.close()
     want = model.forward_logits(params, ids, B, T).reshape(B, T, V)[:, -1]
     assert np.abs(got - want).max() <= 1e-4 * np.abs(want).max()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0)])
+@pytest.mark.parametrize("M,N,K,wg", [(1, 1, 1200, 8), (65, 63, 8190, 48), (127, 2050, 777, 198),
+                                      (16 * 64, 16 * 64, 1201, 0), (16 * 64 + 1, 16 * 64, 1201, 0),
+                                      (1000, 4, 8190, 256), (4097, 200, 64, 0)])
+def test_lone_workgroups(dev, M, N, K, ta, tb, wg):
+    """The plan's own kernel up to and just beyond one 64x64 workgroup per CU
+    (256), with and without split-K: fp32 tiles up to it, split products beyond."""
+    dev.current()
+    rng = np.random.default_rng(M + 3 * N + 7 * K + ta + 2 * tb)
+    A = rng.standard_normal((M, K)).astype(np.float32)
+    B = rng.standard_normal((K, N)).astype(np.float32)
+    dA, lda, dB, ldb = operands(dev, A, B, ta, tb)
+    dC = dev.upload(np.full((M, N), 7.0, np.float32))
+    try:
+        dev.matmul(ta, tb, dA, dB, dC, M, N, K, lda, ldb, N)
+        name, splits = dev.last_variant()
+        got = dev.download(dC, (M, N))
+    finally:
+        for p in (dA, dB, dC):
+            dev.free(p)
+    if wg:
+        assert -(-M // 64) * -(-N // 64) * splits == wg, (name, splits)
+    want = A.astype(np.float64) @ B.astype(np.float64)
+    bound = (K + 8) * U * (np.abs(A).astype(np.float64) @ np.abs(B).astype(np.float64))
+    assert (np.abs(got - want) <= bound).all(), (name, float((np.abs(got - want) / bound).max()))

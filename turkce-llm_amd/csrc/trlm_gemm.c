@@ -228,7 +228,10 @@ static void select_plan(int M, int N, int K, u32 batch, int* tile, int* splits) 
      * loop is latency-bound (0.75 us per 32-deep step alone on its CU), so
      * split K down to 64-deep chunks over up to 8 partitions, 128-deep up to
      * 16 and 256-deep beyond, two workgroups per CU at most.  Measured on
-     * MI355X against at most 8: 17x1374x7742 35.3 -> 27.2 us (16). */
+     * MI355X against at most 8: 17x1374x7742 35.3 -> 27.2 us (16).  One
+     * workgroup per CU where that leaves chunks of at most 512: the fp32
+     * tile's case (see trlm_gemm_ws), 36x3795x1091 16.2 (7 splits) -> 14.3 us
+     * (4), 3644x63x1428 19.2 (8) -> 16.7 (4). */
     if ((M <= 128 || N <= 128) && batch == 1) {
         long long tiles = (long long)cdiv(M, 64) * cdiv(N, 64);
         if (tiles < 128) {
@@ -236,7 +239,8 @@ static void select_plan(int M, int N, int K, u32 batch, int* tile, int* splits) 
             if (smax > 8) smax = 8;
             if (smax < K / 128) smax = K / 128 < 16 ? K / 128 : 16;
             if (smax < K / 256) smax = K / 256;
-            if (smax > 2 * CUS / tiles) smax = 2 * CUS / tiles;
+            const long long per_cu = (long long)K * tiles <= 512ll * CUS ? 1 : 2;
+            if (smax > per_cu * CUS / tiles) smax = per_cu * CUS / tiles;
             *tile = T_64x64_K32;
             for (size_t j = 0; j < sizeof(PLAN_SPLITS) / sizeof(PLAN_SPLITS[0]); j++)
                 if (PLAN_SPLITS[j] <= smax) *splits = PLAN_SPLITS[j];
@@ -511,6 +515,15 @@ i32 trlm_gemm_ws(TrlmGemm* e, i32 trans_a, i32 trans_b, hipDeviceptr_t A, hipDev
             splits = cdiv(K, kchunk);
         }
     }
+    /* At most one 64x64 workgroup per CU: nothing hides a lone workgroup's
+     * splitting, and the fp32 tile of the same plan is the faster.  MI355X,
+     * split products / fp32 tiles (us): 43x8816x710 TN (138 workgroups) 22.4 /
+     * 17.8, 173x28x7365 TN (24 splits, 72) 16.5 / 13.5, 11x15x1051 NT (7) 10.7
+     * / 9.6; over 46 drawn shapes up to 256 workgroups 0.79 to 1.02 of the
+     * time, 257 to 320 0.95 to 1.08, beyond them 1.00 to 1.29. */
+    if (aligned && tile == T_64x64_K32 && e->force_tile < 0 &&
+        (long long)p.tiles_m * p.tiles_n * (splits > 1 ? (u32)splits : batch) <= CUS)
+        kernel = e->k[layout][tile];
     snprintf(e->last, sizeof(e->last), "k_gemm_%s_%s", LAYOUT_NAME[layout],
              aligned ? TILES[tile].name : tile == T_128x128 ? "128x128_u" : "64x64_u");
     e->last_splits = splits;
