@@ -1,12 +1,15 @@
 """The split-product GEMMs (gemm_split.hip): every fp32 operand as three bf16
 parts, six products on the bf16 matrix cores.
 
-  - the split itself, restated in numpy: the three parts add up to the operand
-    exactly and the products left out are below 2^-24 of the whole;
+  - the split itself, restated in numpy: the three parts add up to 2^24 times
+    the operand exactly, from the smallest subnormal to 2^103, none of them is
+    subnormal, and the products left out are below 2^-24 of the whole;
   - each variant at the edges of its tiles and k steps, componentwise within
     the bound of a sum of K rounded products, (K + 8) 2^-24 sum |a||b|;
   - sums over C's rows with operands of one sign: what the matrix cores' own
     rounding would leave in all rows alike is no more than the fp32 variant's;
+  - the same bound for operands down to the smallest subnormals against large
+    ones, and for operands and sums beyond what the scaled split holds;
   - infinities, NaN and magnitudes that bf16 rounds to infinity come out as
     fp32 gives them, and padding past N never reaches C;
   - the SwiGLU epilogues agree with the oracle through the decoder's prefill.
@@ -26,14 +29,15 @@ def bf16(x):
 
 def test_three_parts_add_up_exactly():
     rng = np.random.default_rng(0)
-    x = np.ldexp(rng.uniform(1, 2, 200000), rng.integers(-100, 120, 200000)).astype(np.float32)
-    x *= rng.choice(np.float32([-1, 1]), x.size)
+    x = np.ldexp(rng.uniform(1, 2, 200000), rng.integers(-149, 103, 200000)).astype(np.float32)
+    x *= rng.choice(np.float32([-1, 1]), x.size) * np.float32(2.0 ** 24)
     h = bf16(x)
     m = bf16(x - h)
     low = (x - h) - m
     assert np.array_equal(bf16(low), low)            # the last part is a bf16 as it stands
     s = h.astype(np.float64) + m + low
     assert np.array_equal(s, x.astype(np.float64))
+    assert all((np.abs(v[v != 0]) >= 2.0 ** -126).all() for v in (h, m, low))
     a, b = slice(0, 100000), slice(100000, 200000)
     H, M, L = [v.astype(np.float64) for v in (h, m, low)]
     left = np.abs(M[a] * L[b]) + np.abs(L[a] * M[b]) + np.abs(L[a] * L[b])
@@ -133,6 +137,25 @@ def test_row_sums_keep_no_common_error(dev, tile):
         got = product(dev, t, 4, A, B, 0, 0).astype(np.float64).sum(0)
         err[t] = np.linalg.norm(got - want) / np.linalg.norm(want)
     assert err[tile] <= 4 * err["256x128"] + U, err
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tile", SPLIT_TILES)
+@pytest.mark.parametrize("ea,eb", [(-111, 90), (-115, 100), (100, -120), (-126, 103), (103, -126), (-149, 103),
+                                   (103, -140), (-60, -60), (110, -100), (-126, 120), (50, 60)])
+def test_ends_of_the_range(dev, tile, ea, eb):
+    """Operands around 2^ea and 2^eb: 24 bits of each count, down to the
+    subnormals (-126 and below; an operand of -149 has its one bit), up to the
+    split's 2^104, and past it and past sums of 2^80 (the last three)."""
+    rng = np.random.default_rng(1000 + ea + 3 * eb)
+    M, N, K = 130, 67, 77
+    A = np.ldexp(rng.choice([-1.0, 1.0], (M, K)) * rng.uniform(1, 2, (M, K)), ea).astype(np.float32)
+    B = np.ldexp(rng.choice([-1.0, 1.0], (K, N)) * rng.uniform(1, 2, (K, N)), eb).astype(np.float32)
+    want = A.astype(np.float64) @ B.astype(np.float64)
+    bound = (K + 8) * U * (np.abs(A).astype(np.float64) @ np.abs(B).astype(np.float64)) + 2.0 ** -149
+    for ta, tb in ((0, 0), (0, 1), (1, 0)):
+        got = product(dev, tile, 1, A, B, ta, tb)
+        assert (np.abs(got - want) <= bound).all(), (ta, tb, float((np.abs(got - want) / bound).max()))
 
 
 @pytest.mark.gpu

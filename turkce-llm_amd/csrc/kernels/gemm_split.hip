@@ -1,10 +1,22 @@
 // gemm_split.hip -- fp32 GEMMs on the bf16 matrix cores, without loss of
-// precision: every fp32 operand is split into three bf16 parts that add up
-// to it exactly, and the products that matter are formed on
+// precision: every fp32 operand, times 2^24, is split into three bf16 parts
+// that add up to it exactly, and the products that matter are formed on
 // v_mfma_f32_32x32x16_bf16 with fp32 accumulation.
 //
-//   x = h + m + l,  h = bf16(x), m = bf16(x - h), l = x - h - m  (exact)
-//   a*b ~ al*bh + ah*bl + am*bm + am*bh + ah*bm + ah*bh
+//   2^24 x = h + m + l,  h = bf16(2^24 x), m = bf16(2^24 x - h), l = the rest (exact)
+//   2^48 a*b ~ al*bh + ah*bl + am*bm + am*bh + ah*bm + ah*bh
+//
+// The factor is there for the smallest operands: the lowest bit of any fp32
+// (2^-149) becomes 2^-125, so no part is ever subnormal.  Without it the
+// split held 24 bits only from 2^-110 on and 8 at 2^-126.  Sums are scaled
+// back by 2^-48.  Operands near 2^104 and sums near 2^80 and beyond overflow
+// and take the recomputation on the fp32 matrix cores that an infinity takes.
+// It costs one multiplication per value of B (A's replaces its sign change):
+// QKV 8192x1152x384 58.3 -> 59.0 us, the LM head unchanged; the same bits.
+//
+// Sums of products of bf16 parts: Henry, Tang and Heinecke, "Leveraging the
+// bfloat16 Artificial Intelligence Datatype For Higher-Precision
+// Computations", ARITH 2019.
 //
 // The three products left out are below 2^-24 of |a*b|, and a product of two
 // bf16 has 16 significant bits, so it enters the sum unrounded: what is
@@ -40,13 +52,12 @@ typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
 
-// The three bf16 parts of eight floats, their signs flipped where sign is
-// 0x80000000, two to a register.
-__device__ __forceinline__ void split8(const float (&x)[8], unsigned sign, u32x4& h, u32x4& m, u32x4& l) {
+// The three bf16 parts of eight floats times scale (a power of two, of either
+// sign), two to a register.
+__device__ __forceinline__ void split8(const float (&x)[8], float scale, u32x4& h, u32x4& m, u32x4& l) {
 #pragma unroll
     for (int i = 0; i < 4; i++) {
-        const float x0 = __builtin_bit_cast(float, __builtin_bit_cast(unsigned, x[2 * i]) ^ sign);
-        const float x1 = __builtin_bit_cast(float, __builtin_bit_cast(unsigned, x[2 * i + 1]) ^ sign);
+        const float x0 = x[2 * i] * scale, x1 = x[2 * i + 1] * scale;
         const unsigned hu = __builtin_bit_cast(unsigned, __builtin_convertvector((f32x2){x0, x1}, bf16x2));
         const float r0 = x0 - __builtin_bit_cast(float, hu << 16);
         const float r1 = x1 - __builtin_bit_cast(float, hu & 0xffff0000u);
@@ -61,6 +72,7 @@ __device__ __forceinline__ void split8(const float (&x)[8], unsigned sign, u32x4
 
 constexpr int X3_BK = 32;     // k per step
 constexpr int X3_FLIP = 4;    // steps between changes of the sum's sign
+constexpr float X3_SCALE = 0x1p24f, X3_UNSCALE = 0x1p-48f;   // of an operand, of a sum
 
 // One operand's part of a k step: R rows (of m or n) by 32 k.
 // LDS: [plane h/m/l][chunk c of 8 k][slot], 16 bytes each; chunk c holds
@@ -152,7 +164,7 @@ struct X3Tile {
             }
         }
     }
-    __device__ __forceinline__ void store(u32x4* lds, unsigned sign) const {
+    __device__ __forceinline__ void store(u32x4* lds, float scale) const {
 #pragma unroll
         for (int i = 0; i < NI; i++) {
             const int id = threadIdx.x + 256 * i;
@@ -161,7 +173,7 @@ struct X3Tile {
 #pragma unroll
             for (int w = 0; w < W; w++) {
                 u32x4 h, m, l;
-                split8(x[W * i + w], sign, h, m, l);
+                split8(x[W * i + w], scale, h, m, l);
                 u32x4* d = lds + c * COL + slot(r + w);
                 d[0] = h;
                 d[4 * COL] = m;
@@ -237,8 +249,8 @@ __device__ __forceinline__ void gemm_epilogue_glu2(const GemmParams& p, const f3
 
 // A wave block recomputed on the fp32 matrix cores, straight from global
 // memory.  Only for a block with an infinity or NaN in it: an operand that is
-// infinite (or rounds to infinity in bf16) has no split, and its products
-// must come out as fp32 gives them.
+// infinite (or is once scaled, or rounds to infinity in bf16) has no split,
+// and its products must come out as fp32 gives them.
 template <int TA, int TB, int FM, int FN, bool ILA, bool ILB, class ColB>
 __device__ __forceinline__ void gemm_wave_f32(const GemmParams& p, const float* A, const float* B, int r0,
                                               ColB col, int kb, int ke, int lane, f32x16 (&acc)[FM][FN]) {
@@ -330,23 +342,23 @@ __device__ __forceinline__ void gemm_x3_body(const GemmParams& p) {
     // all of them and would show in sums over C's rows (a bias gradient's), so
     // the sum is formed negated for every other four steps: two steps
     // positive, four negative, four positive, ...
-    unsigned sign = 0;
-    auto flip = [&] {
-        sign ^= 0x80000000u;
+    float scale = X3_SCALE;
+    auto times = [&](float f) {
 #pragma unroll
         for (int i = 0; i < FM; i++)
 #pragma unroll
             for (int j = 0; j < FN; j++)
 #pragma unroll
-                for (int r = 0; r < 16; r++) acc[i][j][r] = -acc[i][j][r];
+                for (int r = 0; r < 16; r++) acc[i][j][r] *= f;
     };
     for (int t = 0; t < nk; t++) {
         if (t % X3_FLIP == X3_FLIP / 2) {
             asm volatile("");   // a branch, not a select per element in every step
-            flip();
+            scale = -scale;
+            times(-1.f);
         }
-        ta.store(la, sign);
-        tb.store(lb, 0);
+        ta.store(la, scale);
+        tb.store(lb, X3_SCALE);
         if (TB == 0 && cs_on) {
 #pragma unroll
             for (int i = 0; i < CW; i++)
@@ -375,7 +387,7 @@ __device__ __forceinline__ void gemm_x3_body(const GemmParams& p) {
         }
         __syncthreads();
     }
-    if (sign) flip();
+    times(scale > 0.f ? X3_UNSCALE : -X3_UNSCALE);
     if (TB == 0 && cs_on) {
         // the four chunks' threads of a column, in chunk order
         float* xs = (float*)lds;
