@@ -546,17 +546,11 @@ TILE_DIMS = {"256x128": (256, 128), "128x256": (128, 256), "128x128": (128, 128)
              "64x128": (64, 128), "64x128_k32": (64, 128), "64x64": (64, 64), "64x64_k32": (64, 64)}
 
 
-# The trainer's engines keep the fp32 tiles: their plan (tile, split-K) at B8 T1024.
-TRAINER_PLAN = {"LM-head fwd": ("128x128", 1), "LM-head dX": ("128x128", 8), "LM-head dW": ("128x128", 1),
-                "QKV dW": ("64x64_k32", 7), "attn-out dW": ("64x64_k32", 7), "gate_up dW": ("64x64_k32", 4),
-                "down dW": ("64x64_k32", 8)}
-
-
 def gemm_roles():
     """(kernel, total work-items) -> role for the B8 T1024 training step's
-    GEMMs (and their split-K reductions), from the trainer's plan (64x64_k32
-    without a split where TRAINER_PLAN has no entry); launches are tiles x 256
-    work-items x splits."""
+    GEMMs (and their split-K reductions), from the plan of the trainer's
+    engines, which keep to fp32; launches are tiles x 256 work-items x splits."""
+    trlm = load_trlm()
     shapes = [("QKV fwd", 0, 0, M, 3 * D, D), ("attn-out fwd", 0, 0, M, D, D), ("gate_up fwd", 0, 0, M, 2 * F, D),
               ("down fwd", 0, 0, M, D, F), ("LM-head fwd", 0, 1, M, V, D), ("QKV dX", 0, 1, M, D, 3 * D),
               ("attn-out dX", 0, 1, M, D, D), ("gate_up dX", 0, 1, M, D, 2 * F), ("down dX", 0, 1, M, F, D),
@@ -564,9 +558,8 @@ def gemm_roles():
               ("gate_up dW", 1, 0, D, 2 * F, M), ("down dW", 1, 0, F, D, M), ("LM-head dW", 1, 0, V, D, M)]
     roles = {}
     for role, ta, tb, m, n, k in shapes:
-        tile, splits = TRAINER_PLAN.get(role, ("64x64_k32", 1))
-        name = "k_gemm_%s_%s" % ("tn" if ta else "nt" if tb else "nn", tile)
-        bm, bn = TILE_DIMS[tile]
+        name, splits = trlm.gemm_plan(ta, tb, m, n, k, fp32=True, glu_F=F if role == "gate_up fwd" else 0)
+        bm, bn = TILE_DIMS[name.split("_", 3)[3].replace("_glu", "")]
         grid = -(-m // bm) * -(-n // bn) * 256 * splits
         roles.setdefault((name[:40], str(grid)), []).append(role)
         if splits > 1:

@@ -70,11 +70,23 @@ void trlm_gemm(TrlmGemm* e, i32 trans_a, i32 trans_b, hipDeviceptr_t A, hipDevic
 i32 trlm_gemm_noalloc(TrlmGemm* e, i32 trans_a, i32 trans_b, hipDeviceptr_t A, hipDeviceptr_t B, hipDeviceptr_t C,
                       i32 M, i32 N, i32 K, i32 lda, i32 ldb, i32 ldc, u32 batch, i64 sA, i64 sB, i64 sC,
                       f32 alpha, f32 beta, hipDeviceptr_t bias, hipDeviceptr_t resid, i32 ldr);
-/* Name of the kernel variant and split-K factor the last trlm_gemm call used. */
+/* Keeps the engine to the fp32 matrix cores from here on, as a trainer's
+ * engines are: the tiles and plan of k_gemm_*, and k_smallgemm_*.  Without it
+ * an engine takes products of exact bf16 splits (k_xgemm_*) where they are
+ * the faster. */
+void trlm_gemm_keep_fp32(TrlmGemm* e);
+/* Name of the kernel and split-K factor the last trlm_gemm call used: the
+ * fp32 tiles k_gemm_<layout>_<tile>, the split products
+ * k_xgemm_<layout>_<tile>, or k_smallgemm_<layout> (which shares k out inside
+ * a workgroup: no split-K, 1); "_u" for unaligned operands. */
 const char* trlm_gemm_last_variant(TrlmGemm* e, i32* splits);
-/* The variant and split-K factor trlm_gemm picks for 16-byte-aligned operands
+/* The kernel and split-K factor trlm_gemm picks for 16-byte-aligned operands
  * of this shape (host-only; no device call). */
 const char* trlm_gemm_plan(i32 trans_a, i32 trans_b, i32 M, i32 N, i32 K, u32 batch, i32* splits);
+/* The same for another engine or product: fp32 != 0, an engine kept to fp32;
+ * glu_F > 0, the gate/up product with its SwiGLU (NN, N = 2 glu_F). */
+const char* trlm_gemm_plan_ex(i32 trans_a, i32 trans_b, i32 M, i32 N, i32 K, u32 batch, i32 fp32, i32 glu_F,
+                              i32* splits);
 /* Tuning hook: make later calls on this engine use the named aligned tile
  * variant ("256x128", "128x256", "128x128", "128x128_k32", "64x128",
  * "64x128_k32", "64x64", "64x64_k32") and, when splits > 0, that split-K

@@ -123,6 +123,10 @@ def test_code_object_has_every_kernel(trlm):
     names |= {"k_gemm_%s_%s" % (l, t) for l in ("nn", "nt", "tn") for t in (
         "256x128", "128x256", "128x128", "128x128_k32", "64x128", "64x128_k32", "64x64", "64x64_k32")}
     names |= {"k_gemm_%s_64x64_u" % l for l in ("nn", "nt", "tn", "tt")} | {"k_gemm_nn_64x64_k32_glu"}
+    names |= {"k_xgemm_%s_%s" % (l, t) for l in ("nn", "nt", "tn") for t in ("128x128", "64x128_k32", "64x64_k32",
+                                                                             "64x64_u", "128x128_u")}
+    names |= {"k_xgemm_tt_64x64_u", "k_xgemm_nn_64x64_k32_glu", "k_xgemm_nn_128x128_glu", "k_smallgemm_nn_glu"}
+    names |= {"k_smallgemm_%s%s" % (l, u) for l in ("nn", "nt", "tn") for u in ("", "_u")}
     for n in sorted(names):
         assert n.encode() + b"\0" in blob, n
 
@@ -156,13 +160,15 @@ def test_kernel_argument_blocks_match_host_structs(trlm, tmp_path):
     want = {}
     for k in kernels:
         n = k[".name"]
-        if n.startswith("k_gemm_") and not n.startswith("k_gemm_splitk"):
+        if re.match(r"k_(x|small)?gemm_", n) and not n.startswith("k_gemm_splitk"):
             want[n] = gemm
         elif re.match(r"k_attn_(fwd|bwd_dkv|bwd_dq|dvec)_hd\d+$", n):
             want[n] = attn
         elif n in ("k_dec_out", "k_dec_gu", "k_dec_down") or re.match(r"k_dec_(qkv_attn_hd|head_k)\d+$", n):
             want[n] = dec
     assert len([n for n in want if n.startswith("k_gemm_")]) == 29   # 8 tiles x 3 layouts, 4 unaligned, SwiGLU
+    assert len([n for n in want if n.startswith("k_xgemm_")]) == 18   # 3 tiles x 3 layouts, 7 unaligned, 2 SwiGLU
+    assert len([n for n in want if n.startswith("k_smallgemm_")]) == 7   # 3 layouts, aligned and not, SwiGLU
     assert len([n for n in want if n.startswith("k_attn_")]) == 12
     assert len([n for n in want if n.startswith("k_dec_")]) == 9   # out, gu, down, head x 3, QKV + attention x 3
     for k in kernels:
@@ -245,15 +251,17 @@ def test_gemm_plan_is_a_pure_function_of_the_shape(trlm):
                 again = hip.trlm_gemm_plan(ta, tb, M, N, K, batch, C.byref(sp)).decode(), sp.value
                 assert first == again
                 name, splits = first
-                assert name.startswith("k_gemm_%s_" % ["nn", "nt", "tn"][ta * 2 + tb]), name
+                assert re.match(r"k_(gemm_%s_|xgemm_%s_|smallgemm_%s$)" % ((["nn", "nt", "tn"][ta * 2 + tb],) * 3),
+                                name), name
                 assert 1 <= splits <= 32
                 if splits > 1:
                     assert batch == 1 and K // splits >= 224, (M, N, K, splits)
-    assert hip.trlm_gemm_plan(1, 1, 64, 64, 64, 1, C.byref(sp)) == b"k_gemm_tt_64x64_u" and sp.value == 1
+    assert hip.trlm_gemm_plan(1, 1, 64, 64, 64, 1, C.byref(sp)) == b"k_xgemm_tt_64x64_u" and sp.value == 1
     # the LM-head forward (15,936 tiles of 128x128, 62 per CU) keeps the
-    # large tile and needs no split
+    # large tile and needs no split, on an engine of its own and on a trainer's
     name = hip.trlm_gemm_plan(0, 1, 8192, 31769, 384, 1, C.byref(sp)).decode()
-    assert name == "k_gemm_nt_128x128" and sp.value == 1
+    assert name == "k_xgemm_nt_128x128" and sp.value == 1
+    assert trlm.gemm_plan(0, 1, 8192, 31769, 384, fp32=True) == ("k_gemm_nt_128x128", 1)
 
 
 def test_attention_job_table(trlm):

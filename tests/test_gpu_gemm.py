@@ -1,4 +1,6 @@
-"""fp32 MFMA GEMM parity through the C ABI (trlm_gemm), against fp64 numpy.
+"""fp32 GEMM parity through the C ABI (trlm_gemm), against fp64 numpy: every
+test on an engine kept to the fp32 tiles (a trainer's kernels) and on one that
+takes the split products.
 
 Covers the reference's GEMM contract (train_kernels.cu:97-193,226-329;
 gpu_train.c:42-118): NN / NT / TN layouts, batched strides, alpha/beta,
@@ -15,11 +17,21 @@ import pytest
 pytestmark = pytest.mark.gpu
 
 
-@pytest.fixture(scope="module")
-def dev(trlm):
-    d = trlm.Device()
+SPLIT_TILES = ("128x128", "64x128_k32", "64x64_k32")   # the tiles that also come from split products
+
+
+@pytest.fixture(scope="module", params=["fp32", "split"])
+def dev(trlm, request):
+    d = trlm.Device(fp32=request.param == "fp32")
+    d.fp32 = request.param == "fp32"
     yield d
     d.close()
+
+
+def kernel(dev, ta, tb, tile):
+    """The kernel of a forced tile on this engine."""
+    return "k_%s_%s_%s" % ("xgemm" if not dev.fp32 and tile in SPLIT_TILES else "gemm",
+                           ["nn", "nt", "tn"][ta * 2 + tb], tile)
 
 
 def stored(op_mat, trans):
@@ -210,7 +222,7 @@ def test_gemm_epilogue_terms_bitwise(dev, tile, ta, tb):
         for splits in (1, 3):
             dev.force(tile, splits)
             P, var = run_gemm(dev, A, B, ta, tb, alpha=0.5)
-            assert var == ("k_gemm_%s_%s" % (["nn", "nt", "tn"][ta * 2 + tb], tile), splits), var
+            assert var == (kernel(dev, ta, tb, tile), splits), var
             ok, rel = close(P, ref64(A, B, 0.5))
             assert ok, (var, rel)
             cases = [(dict(bias=bias), P + bias), (dict(resid=resid), resid + P),
@@ -377,7 +389,7 @@ def test_gemm_every_tile_variant(dev, tile, ta, tb):
         for splits in (1, 3):
             dev.force(tile, splits)
             got, var = run_gemm(dev, A, B, ta, tb, alpha=0.5, beta=1.0, C0=C0, bias=bias, resid=resid)
-            assert var == ("k_gemm_%s_%s" % (["nn", "nt", "tn"][ta * 2 + tb], tile), splits), var
+            assert var == (kernel(dev, ta, tb, tile), splits), var
             ok, rel = close(got, ref64(A, B, 0.5, 1.0, C0, bias, resid))
             assert ok, (var, rel)
     finally:
@@ -465,7 +477,7 @@ def test_gemm_store_paths_agree(dev, tile, ta, tb):
                 elif terms == "beta":
                     kw = dict(beta=1.0)
                 dev.matmul(ta, tb, dA, dB, dC, M, N, K, As.shape[1], Bs.shape[1], ldc, alpha=0.5, **kw)
-                assert dev.last_variant() == ("k_gemm_%s_%s" % (["nn", "nt", "tn"][ta * 2 + tb], tile), 1)
+                assert dev.last_variant() == (kernel(dev, ta, tb, tile), 1)
                 got = dev.download(dC, (M, ldc))
                 outs.append((got, C0))
                 dev.free(dC)

@@ -1,4 +1,4 @@
-"""The small-product GEMMs (gemm_small.hip, reported as 32x32): one 32x32 tile
+"""The small-product GEMMs (gemm_small.hip, k_smallgemm_*): one 32x32 tile
 of C per workgroup, k shared out over its four waves.
 
 Each layout, aligned and not, at the edges of its tile and of its 32-deep
@@ -48,7 +48,7 @@ def test_edges_and_epilogue(dev, M, N, K, ta, tb, pad):
     finally:
         for p in (dA, dB, dC, dR, db):
             dev.free(p)
-    assert "32x32" in name and splits == min(4, -(-K // 32))
+    assert (name, splits) == ("k_smallgemm_" + ["nn", "nt", "tn"][2 * ta + tb] + ("" if pad else "_u"), 1)
     prod = 0.5 * (A.astype(np.float64) @ B.astype(np.float64))
     want = R + ((prod + 2.0 * C0) + bias)
     mag = 0.5 * (np.abs(A).astype(np.float64) @ np.abs(B).astype(np.float64))

@@ -62,7 +62,8 @@ def product(dev, tile, splits, A, B, ta, tb, fill=0.0):
     try:
         dev.force(tile, splits)
         dev.matmul(ta, tb, dA, dB, dC, M, N, K, lda, ldb, N)
-        assert dev.last_variant()[0].endswith(tile)
+        family = "xgemm" if tile in SPLIT_TILES else "gemm"
+        assert dev.last_variant() == ("k_%s_%s_%s" % (family, ["nn", "nt", "tn"][2 * ta + tb], tile), splits)
         return dev.download(dC, (M, N))
     finally:
         dev.force(None)
@@ -95,7 +96,7 @@ def test_edges(dev, tile, ta, tb, M, N, K, splits):
 @pytest.mark.gpu
 @pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0), (1, 1)])
 @pytest.mark.parametrize("M,N,K,splits", [(1, 1, 1, 1), (129, 63, 31, 1), (63, 131, 33, 1), (257, 67, 447, 2),
-                                          (2051, 4099, 37, 1)])
+                                          (2051, 4099, 37, 1), (3001, 4001, 131, 1)])
 def test_unaligned_edges(dev, M, N, K, ta, tb, splits):
     """Tight odd rows (64x64_u, and 128x128_u for the last shape): every value
     is loaded by itself and none past the last row's end (an odd M or N leaves
@@ -115,7 +116,8 @@ def test_unaligned_edges(dev, M, N, K, ta, tb, splits):
         for p in (dA, dB, dC):
             dev.free(p)
     if As.shape[1] % 4 or Bs.shape[1] % 4:
-        assert name.endswith("_u")
+        assert name == "k_xgemm_%s_%s_u" % (["nn", "nt", "tn", "tt"][2 * ta + tb],
+                                            "128x128" if M == 3001 and not (ta and tb) else "64x64")
     want = A.astype(np.float64) @ B.astype(np.float64)
     bound = (K + 8) * U * (np.abs(A).astype(np.float64) @ np.abs(B).astype(np.float64))
     assert (np.abs(got - want) <= bound).all(), (name, float((np.abs(got - want) / np.maximum(bound, 1e-30)).max()))
@@ -213,8 +215,8 @@ def test_swiglu_epilogue_of_both_tiles(trlm, orc, F, B, T):
 @pytest.mark.gpu
 @pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0)])
 @pytest.mark.parametrize("M,N,K,wg", [(1, 1, 1200, 8), (65, 63, 8190, 48), (127, 2050, 777, 198),
-                                      (16 * 64, 16 * 64, 1201, 0), (16 * 64 + 1, 16 * 64, 1201, 0),
-                                      (1000, 4, 8190, 256), (4097, 200, 64, 0)])
+                                      (16 * 64, 16 * 64, 1201, 256), (16 * 64 + 1, 16 * 64, 1201, 17 * 16 * 4),
+                                      (1000, 4, 8190, 256), (4097, 200, 64, 260)])
 def test_lone_workgroups(dev, M, N, K, ta, tb, wg):
     """The plan's own kernel up to and just beyond one 64x64 workgroup per CU
     (256), with and without split-K: fp32 tiles up to it, split products beyond."""
@@ -231,8 +233,9 @@ def test_lone_workgroups(dev, M, N, K, ta, tb, wg):
     finally:
         for p in (dA, dB, dC):
             dev.free(p)
-    if wg:
-        assert -(-M // 64) * -(-N // 64) * splits == wg, (name, splits)
+    ran = -(-M // 64) * -(-N // 64) * splits
+    assert ran == wg, (name, splits)
+    assert name == "k_%s_%s_64x64_k32" % ("gemm" if ran <= 256 else "xgemm", ["nn", "nt", "tn"][2 * ta + tb])
     want = A.astype(np.float64) @ B.astype(np.float64)
     bound = (K + 8) * U * (np.abs(A).astype(np.float64) @ np.abs(B).astype(np.float64))
     assert (np.abs(got - want) <= bound).all(), (name, float((np.abs(got - want) / bound).max()))

@@ -3,16 +3,17 @@ fixed 32 MiB scratch array instead of an allocated workspace.
 
 Through the C ABI:
   - two calls in a row -- a weight-gradient shape that takes split-K
-    (384x1152x8192 TN: 7 splits, 12.4 MB of partials), then a smaller
-    decode-sized one with the full epilogue (64 rows, alpha, beta*C, bias,
-    residual) -- each equal to trlm_gemm's result on the same inputs bit for
-    bit (same plan, same kernels), with the device's free memory unchanged;
+    (384x1152x8192 TN: 16 splits, 28 MB of partials), then a smaller
+    decode-sized one with the full epilogue (64x1152x1536: 12 splits, 3.5 MB;
+    alpha, beta*C, bias, residual) -- each equal to trlm_gemm's result on the
+    same inputs bit for bit (same plan, same kernels), with the device's free
+    memory unchanged;
   - the scratch boundary: with 8 splits forced on both engines, a
     1024x1024 product whose partials fill exactly 32 MiB runs with its 8
     splits, and a 1028x1024 one (32 MiB + 128 KiB) runs with the 7 splits
     that fit, each equal bit for bit to trlm_gemm forced to that split count;
-  - the full-size LM-head dX (8192x384x31769 NN, planned with 8 splits,
-    100.7 MB of partials) runs with the 2 splits that fit, equal to
+  - the full-size LM-head dX (8192x384x31769 NN, planned with 12 splits,
+    151 MB of partials) runs with the 2 splits that fit, equal to
     trlm_gemm forced to 2 splits.
 """
 import ctypes as C
@@ -61,7 +62,7 @@ def _lds(c):
 
 def test_noalloc_equals_trlm_gemm_two_calls(trlm):
     rng = np.random.default_rng(7)
-    cases = [_case(rng, 1, 0, 384, 1152, 8192, False), _case(rng, 0, 0, 64, 1152, 384, True)]
+    cases = [_case(rng, 1, 0, 384, 1152, 8192, False), _case(rng, 0, 0, 64, 1152, 1536, True)]
     ref = trlm.Device()       # trlm_gemm (allocating engine) on its own context
     dev = trlm.Device()       # trlm_gemm_noalloc on a fresh engine
     try:
@@ -77,6 +78,7 @@ def test_noalloc_equals_trlm_gemm_two_calls(trlm):
             plans.append(ref.last_variant())
         # both take split-K (use the scratch), the second call's partials fewer
         assert plans[0][1] > 1 and plans[1][1] > 1, plans
+        assert not any(name.startswith("k_smallgemm") for name, _ in plans), plans
         assert plans[1][1] * cases[1]["M"] * cases[1]["N"] < plans[0][1] * cases[0]["M"] * cases[0]["N"], plans
         dev.current()
         bufs = []

@@ -1,4 +1,5 @@
-/* trlm_gemm.c -- host dispatch of the fp32 MFMA GEMM kernels (gemm.hip).
+/* trlm_gemm.c -- host dispatch of the fp32 GEMM kernels (gemm.hip, gemm_split.hip,
+ * gemm_small.hip).
  *
  * Plays the role of the reference's gemm()/gemm1()/bf16_gemm*() launch
  * helpers (model/gpu_train.c:42-118): same operand conventions (NN, NT, TN;
@@ -29,9 +30,9 @@ enum { L_NN = 0, L_NT = 1, L_TN = 2 };
 static const char* LAYOUT_NAME[4] = { "nn", "nt", "tn", "tt" };
 
 /* Aligned tile variants: name suffix, tile rows/cols, k step of the fp32
- * kernels (gemm.hip).  128x128, 64x128_k32 and 64x64_k32 also come from exact
- * three-way bf16 splits (gemm_split.hip, k step 32), which an engine takes
- * for them unless it keeps to fp32. */
+ * kernels (gemm.hip, k_gemm_*).  128x128, 64x128_k32 and 64x64_k32 also come
+ * from exact three-way bf16 splits (gemm_split.hip, k_xgemm_*, k step 32),
+ * which an engine takes for them unless it keeps to fp32. */
 typedef struct TileDef { const char* name; int bm, bn, bk; } TileDef;
 enum { T_256x128, T_128x256, T_128x128, T_128x128_K32, T_64x128, T_64x128_K32, T_64x64, T_64x64_K32, T_COUNT };
 static const TileDef TILES[T_COUNT] = {
@@ -105,11 +106,12 @@ TrlmGemm* trlm_gemm_create(HipCtx* ctx) {
 }
 
 /* The engine's products keep to the fp32 matrix cores, with the tiles and
- * split-K of the fp32 plan.  The trainer's engines do: a training run's bits
- * are those of the fp32 tiles, and an optimizer's first steps magnify any
+ * split-K of the fp32 plan (products of few tiles take k_smallgemm_*, which is
+ * fp32 too).  The trainer's engines do: an optimizer's first steps magnify any
  * other rounding, however small (AdamW divides by the gradient's size: after
  * one step of the 12-layer model two correct roundings of it, each 1.7e-6 or
- * less from 64 bits, have gradients 7e-6 to 2e-5 apart). */
+ * less from 64 bits, have gradients 7e-6 to 2e-5 apart), and the evaluation's
+ * loss is bit for bit the training step's, so its products go with them. */
 void trlm_gemm_keep_fp32(TrlmGemm* e) { e->fp32 = 1; }
 
 void trlm_gemm_destroy(TrlmGemm* e) {
@@ -334,8 +336,8 @@ static void select_fp32(int M, int N, int K, u32 batch, int* tile, int* splits) 
         }
 }
 
-/* Products of few tiles (gemm_small.hip, reported as the tile 32x32): one
- * 32x32 tile per workgroup, k shared out over its waves.  Up to two tiles per
+/* Products of few tiles (gemm_small.hip, k_smallgemm_*): one 32x32 tile per
+ * workgroup, k shared out over its waves.  Up to two tiles per
  * CU, measured on MI355X against the planned tile (us): 64x1152x384 5.8 / 8.0,
  * 128x2048x384 (256 tiles) 6.1 / 9.9, 512x384x384 (192) 6.0 / 11.9,
  * 512x1024x384 (512) 9.9 / 10.8, but 512x1152x384 (576) 12.4 / 12.2; with less
@@ -351,26 +353,109 @@ static int small_gemm(int M, int N, int K, u32 batch, int aligned) {
     return batch == 1 && K <= (M > 128 && N > 128 ? 1152 : 768) && tiles <= most;
 }
 
-/* How many ways its waves share out k: up to four, 32 k at a time. */
-static int small_splits(int K) { return K > 96 ? 4 : K > 32 ? cdiv(K, 32) : 1; }
+#define ANY_ROOM (~0ull)   /* a workspace that grows */
+
+/* What runs a product: the kernel's family and tile, the split-K factor and
+ * each split's share of k. */
+enum { FP32, SPLIT, SMALL };
+typedef struct Plan { int family, tile, splits, kchunk; } Plan;
+
+/* What a product asks of its plan beside its shape. */
+typedef struct PlanOpts {
+    int aligned;                /* 16-byte rows */
+    int fp32;                   /* keeps to the fp32 tiles */
+    int stats, whole;           /* row statistics; an epilogue that needs whole sums (stats, RoPE) */
+    int force_tile, force_splits;
+    u64 slab, ws_floats;        /* floats of one split's partials, and that there is room for */
+} PlanOpts;
+
+/* Shares k out over `splits`, each a multiple of KCHUNK_ALIGN. */
+static void set_splits(Plan* p, int K, int splits) {
+    p->splits = splits;
+    p->kchunk = K;
+    if (splits > 1) {
+        p->kchunk = cdiv(cdiv(K, splits), KCHUNK_ALIGN) * KCHUNK_ALIGN;
+        p->splits = cdiv(K, p->kchunk);
+    }
+}
+
+static Plan make_plan(int layout, int M, int N, int K, u32 batch, const PlanOpts* o) {
+    Plan p = { FP32, T_64x64_K32, 1, K };
+    if (layout != 3 && !o->stats && o->force_tile < 0 && o->force_splits == 0 &&
+        small_gemm(M, N, K, batch, o->aligned)) {
+        p.family = SMALL;
+        return p;
+    }
+    int splits;
+    if (o->fp32) select_fp32(M, N, K, batch, &p.tile, &splits);
+    else select_plan(M, N, K, batch, &p.tile, &splits);
+    if (!o->aligned) {
+        /* the unaligned kernels: one fp32 tile without split-K, two of the
+         * split products' tiles */
+        if (o->fp32 || p.tile != T_128x128 || layout == 3 || o->stats) p.tile = T_64x64_K32;
+        if (o->fp32 || layout == 3) splits = 1;
+    } else if (o->force_tile >= 0) {
+        p.tile = o->force_tile;
+        splits = batch == 1 ? auto_splits(tiles_of(p.tile, M, N, 1), K) : 1;
+    }
+    if (o->force_splits > 0 && batch == 1 && (o->aligned || (!o->fp32 && layout != 3))) splits = o->force_splits;
+    if (o->whole || K < 2 * KCHUNK_ALIGN) splits = 1;
+    set_splits(&p, K, splits);
+    if (p.splits > 1 && (u64)p.splits * o->slab > o->ws_floats) {
+        /* A fixed workspace that cannot hold the plan's partials: run the
+         * most splits whose partials fit (one split needs none).  The k
+         * chunks are formed as for a forced split count, so the result
+         * equals this engine's trlm_gemm forced to that many splits. */
+        u64 fit = o->ws_floats / o->slab;
+        set_splits(&p, K, fit < 2 ? 1 : (int)fit);
+    }
+    if (!o->fp32 && (!o->aligned || has_split(p.tile))) p.family = SPLIT;
+    /* At most one 64x64 workgroup per CU: nothing hides a lone workgroup's
+     * splitting, and the fp32 tile of the same plan is the faster.  MI355X,
+     * split products / fp32 tiles (us): 43x8816x710 TN (138 workgroups) 22.4 /
+     * 17.8, 173x28x7365 TN (24 splits, 72) 16.5 / 13.5, 11x15x1051 NT (7) 10.7
+     * / 9.6; over 46 drawn shapes up to 256 workgroups 0.79 to 1.02 of the
+     * time, 257 to 320 0.95 to 1.08, beyond them 1.00 to 1.29. */
+    if (o->aligned && p.tile == T_64x64_K32 && o->force_tile < 0 &&
+        tiles_of(p.tile, M, N, p.splits > 1 ? (u32)p.splits : batch) <= CUS)
+        p.family = FP32;
+    return p;
+}
+
+/* The plan of the gate/up product [M, 2F] with the SwiGLU epilogue: the
+ * 128-wide tile where F holds whole half tiles and the plan model finds it
+ * the faster of the two. */
+static Plan make_glu_plan(int M, int F, int K, int fp32) {
+    Plan p = { fp32 ? FP32 : SPLIT, T_64x64_K32, 1, K };
+    if (!fp32 && F % 64 == 0 &&
+        plan_cost(&PLAN_TILES[0], M, 2 * F, K, 1, 1) < plan_cost(&PLAN_TILES[2], M, 2 * F, K, 1, 1))
+        p.tile = T_128x128;
+    return p;
+}
+
+/* The kernel's name in the code object. */
+static void plan_name(char* out, size_t size, const Plan* p, int layout, int aligned, int glu) {
+    const char* l = LAYOUT_NAME[layout];
+    const char* end = glu ? "_glu" : aligned ? "" : "_u";
+    if (p->family == SMALL) snprintf(out, size, "k_smallgemm_%s%s", l, end);
+    else
+        snprintf(out, size, "k_%sgemm_%s_%s%s", p->family == SPLIT ? "x" : "", l,
+                 aligned ? TILES[p->tile].name : p->tile == T_128x128 ? "128x128" : "64x64", end);
+}
+
+const char* trlm_gemm_plan_ex(i32 trans_a, i32 trans_b, i32 M, i32 N, i32 K, u32 batch, i32 fp32, i32 glu_F,
+                              i32* splits) {
+    static __thread char name[48];
+    const int layout = trans_a ? (trans_b ? 3 : L_TN) : (trans_b ? L_NT : L_NN);
+    const PlanOpts o = { .aligned = layout != 3, .fp32 = fp32, .force_tile = -1, .ws_floats = ANY_ROOM };
+    const Plan p = glu_F > 0 ? make_glu_plan(M, glu_F, K, fp32) : make_plan(layout, M, N, K, batch ? batch : 1, &o);
+    plan_name(name, sizeof(name), &p, layout, o.aligned, glu_F > 0);
+    if (splits) *splits = p.splits;
+    return name;
+}
 
 const char* trlm_gemm_plan(i32 trans_a, i32 trans_b, i32 M, i32 N, i32 K, u32 batch, i32* splits) {
-    static __thread char name[48];
-    int layout = trans_a ? (trans_b ? 3 : L_TN) : (trans_b ? L_NT : L_NN);
-    int tile, sp;
-    if (layout == 3) {
-        snprintf(name, sizeof(name), "k_gemm_tt_64x64_u");
-        sp = 1;
-    } else if (small_gemm(M, N, K, batch ? batch : 1, 1)) {
-        snprintf(name, sizeof(name), "k_gemm_%s_32x32", LAYOUT_NAME[layout]);
-        sp = small_splits(K);
-    } else {
-        select_plan(M, N, K, batch ? batch : 1, &tile, &sp);
-        if (sp > 1) sp = cdiv(K, cdiv(cdiv(K, sp), KCHUNK_ALIGN) * KCHUNK_ALIGN);
-        snprintf(name, sizeof(name), "k_gemm_%s_%s", LAYOUT_NAME[layout], TILES[tile].name);
-    }
-    if (splits) *splits = sp;
-    return name;
+    return trlm_gemm_plan_ex(trans_a, trans_b, M, N, K, batch, 0, 0, splits);
 }
 
 void trlm_gemm(TrlmGemm* e, i32 trans_a, i32 trans_b, hipDeviceptr_t A, hipDeviceptr_t B, hipDeviceptr_t C,
@@ -423,16 +508,12 @@ i32 trlm_gemm_ws(TrlmGemm* e, i32 trans_a, i32 trans_b, hipDeviceptr_t A, hipDev
         p.A = (const float*)A; p.B = (const float*)B; p.C = (float*)C; p.bias = (const float*)bias;
         p.M = M; p.N = N; p.K = K; p.lda = lda; p.ldb = ldb; p.ldc = ldc; p.ldr = ldr;
         p.splits = 1; p.kchunk = K; p.alpha = alpha; p.beta = 0.0f;
-        /* the 128-wide tile where F holds whole half tiles and the plan
-         * model finds it the faster of the two */
-        const int wide = !e->fp32 && x->glu_F % 64 == 0 && plan_cost(&PLAN_TILES[0], M, N, K, 1, 1) <
-                                                               plan_cost(&PLAN_TILES[2], M, N, K, 1, 1);
-        const int tile = wide ? 128 : 64;
-        p.tiles_m = cdiv(M, tile); p.tiles_n = cdiv(N, tile);
+        const Plan pl = make_glu_plan(M, x->glu_F, K, e->fp32);
+        p.tiles_m = cdiv(M, TILES[pl.tile].bm); p.tiles_n = cdiv(N, TILES[pl.tile].bn);
         p.glu_h = (float*)x->glu_h; p.glu_F = x->glu_F;
-        snprintf(e->last, sizeof(e->last), "k_gemm_%s_%s_glu", LAYOUT_NAME[L_NN], wide ? "128x128" : "64x64_k32");
+        plan_name(e->last, sizeof(e->last), &pl, L_NN, 1, 1);
         e->last_splits = 1;
-        launch(e->fp32 ? e->glu : wide ? e->xglu128 : e->xglu, &p, 1);
+        launch(pl.family == FP32 ? e->glu : pl.tile == T_128x128 ? e->xglu128 : e->xglu, &p, 1);
         return 0;
     }
     if (csum && (batch != 1 || trans_b)) {
@@ -466,67 +547,26 @@ i32 trlm_gemm_ws(TrlmGemm* e, i32 trans_a, i32 trans_b, hipDeviceptr_t A, hipDev
     int layout = trans_a ? (trans_b ? 3 : L_TN) : (trans_b ? L_NT : L_NN);
     int aligned = layout != 3 && aligned16(A) && aligned16(B) && (lda % 4 == 0) && (ldb % 4 == 0) &&
                   (batch == 1 || ((sA % 4 == 0) && (sB % 4 == 0)));
-    if (layout != 3 && !stats && e->force_tile < 0 && e->force_splits == 0 && small_gemm(M, N, K, batch, aligned)) {
+    /* split-K: raw partials into the workspace, then an ordered reduction;
+     * with column sums each split's slab has one more row, M, for them */
+    const u64 slab = ((u64)M + (csum ? 1u : 0u)) * (u64)N;
+    const PlanOpts o = { aligned, e->fp32, stats != NULL, stats || rope, e->force_tile, e->force_splits, slab,
+                         fixed_ws ? fixed_floats : ANY_ROOM };
+    const Plan pl = make_plan(layout, M, N, K, batch, &o);
+    const int tile = pl.tile, splits = pl.splits;
+    plan_name(e->last, sizeof(e->last), &pl, layout, aligned, 0);
+    e->last_splits = splits;
+    if (pl.family == SMALL) {
         p.tiles_m = cdiv(M, 32); p.tiles_n = cdiv(N, 32);
-        snprintf(e->last, sizeof(e->last), "k_gemm_%s_32x32%s", LAYOUT_NAME[layout], aligned ? "" : "_u");
-        e->last_splits = small_splits(K);
         launch(e->small[!aligned][layout], &p, 1);
         return 0;
     }
-    int tile, splits;
-    if (e->fp32) select_fp32(M, N, K, batch, &tile, &splits);
-    else select_plan(M, N, K, batch, &tile, &splits);
-    if (!aligned) {
-        /* the unaligned kernels: one fp32 tile without split-K, two of the
-         * split products' tiles */
-        if (e->fp32 || tile != T_128x128 || layout == 3 || stats) tile = T_64x64_K32;
-        if (e->fp32 || layout == 3) splits = 1;
-    } else if (e->force_tile >= 0) {
-        tile = e->force_tile;
-        splits = batch == 1 ? auto_splits(tiles_of(tile, M, N, 1), K) : 1;
-    }
-    if (e->force_splits > 0 && batch == 1 && (aligned || (!e->fp32 && layout != 3))) splits = e->force_splits;
-    if (stats || rope) splits = 1;         /* these epilogues need whole sums */
-    hipFunction_t kernel = e->k[layout < 3 ? layout : 0][tile];
-    if (!aligned) kernel = e->fp32 ? e->ku[layout] : tile == T_128x128 ? e->xu128[layout] : e->xu[layout];
-    else if (!e->fp32 && has_split(tile)) kernel = e->x[layout][tile];
+    hipFunction_t kernel;
+    if (!aligned) kernel = pl.family == FP32 ? e->ku[layout] : tile == T_128x128 ? e->xu128[layout] : e->xu[layout];
+    else kernel = (pl.family == SPLIT ? e->x : e->k)[layout][tile];
     p.tiles_m = cdiv(M, TILES[tile].bm);
     p.tiles_n = cdiv(N, TILES[tile].bn);
     if (stats) set_stats(&p, stats, stats_cap, TILES[tile].bn);
-    int kchunk = K;
-    if (splits > 1 && K < 2 * KCHUNK_ALIGN) splits = 1;
-    if (splits > 1) {
-        kchunk = cdiv(cdiv(K, splits), KCHUNK_ALIGN) * KCHUNK_ALIGN;
-        splits = cdiv(K, kchunk);
-    }
-    /* split-K: raw partials into the workspace, then an ordered reduction;
-     * with column sums each split's slab has one more row, M, for them */
-    u64 slab = ((u64)M + (csum ? 1u : 0u)) * (u64)N;
-    if (fixed_ws && splits > 1 && (u64)splits * slab > fixed_floats) {
-        /* A fixed workspace that cannot hold the plan's partials: run the
-         * most splits whose partials fit (one split needs none).  The k
-         * chunks are formed as for a forced split count, so the result
-         * equals this engine's trlm_gemm forced to that many splits. */
-        u64 fit = fixed_floats / slab;
-        splits = fit < 2 ? 1 : (int)fit;
-        kchunk = K;
-        if (splits > 1) {
-            kchunk = cdiv(cdiv(K, splits), KCHUNK_ALIGN) * KCHUNK_ALIGN;
-            splits = cdiv(K, kchunk);
-        }
-    }
-    /* At most one 64x64 workgroup per CU: nothing hides a lone workgroup's
-     * splitting, and the fp32 tile of the same plan is the faster.  MI355X,
-     * split products / fp32 tiles (us): 43x8816x710 TN (138 workgroups) 22.4 /
-     * 17.8, 173x28x7365 TN (24 splits, 72) 16.5 / 13.5, 11x15x1051 NT (7) 10.7
-     * / 9.6; over 46 drawn shapes up to 256 workgroups 0.79 to 1.02 of the
-     * time, 257 to 320 0.95 to 1.08, beyond them 1.00 to 1.29. */
-    if (aligned && tile == T_64x64_K32 && e->force_tile < 0 &&
-        (long long)p.tiles_m * p.tiles_n * (splits > 1 ? (u32)splits : batch) <= CUS)
-        kernel = e->k[layout][tile];
-    snprintf(e->last, sizeof(e->last), "k_gemm_%s_%s", LAYOUT_NAME[layout],
-             aligned ? TILES[tile].name : tile == T_128x128 ? "128x128_u" : "64x64_u");
-    e->last_splits = splits;
     if (splits <= 1) {
         launch(kernel, &p, batch);
         return p.stats ? 2 * p.tiles_n : 0;
@@ -545,7 +585,7 @@ i32 trlm_gemm_ws(TrlmGemm* e, i32 trans_a, i32 trans_b, hipDeviceptr_t A, hipDev
     q.C = (float*)W;
     q.ldc = N;
     q.sW = (long long)slab;
-    q.kchunk = kchunk;
+    q.kchunk = pl.kchunk;
     q.splits = splits;
     q.alpha = 1.0f; q.beta = 0.0f; q.bias = NULL; q.resid = NULL;
     launch(kernel, &q, (u32)splits);
@@ -584,7 +624,7 @@ f32 trlm_timer_stop_ms(TrlmTimer* t) {
     return ms;
 }
 
-const char* trlm_version(void) { return "trlm-mi355x 0.1 (gfx950, fp32 MFMA)"; }
+const char* trlm_version(void) { return "trlm-mi355x 0.1 (gfx950, fp32 and split bf16 MFMA)"; }
 
 u64 trlm_sizeof_gpu_trainer(void) { return (u64)sizeof(GpuTrainer); }
 u64 trlm_sizeof_hip_ctx(void) { return (u64)sizeof(HipCtx); }

@@ -222,6 +222,9 @@ def _bind(host, hip):
     _sig(hip, "trlm_gemm_last_variant", C.c_char_p, [C.c_void_p, C.POINTER(C.c_int32)])
     _sig(hip, "trlm_gemm_plan", C.c_char_p, [C.c_int32, C.c_int32, C.c_int32, C.c_int32, C.c_int32, C.c_uint32,
                                              C.POINTER(C.c_int32)])
+    _sig(hip, "trlm_gemm_plan_ex", C.c_char_p, [C.c_int32, C.c_int32, C.c_int32, C.c_int32, C.c_int32, C.c_uint32,
+                                                C.c_int32, C.c_int32, C.POINTER(C.c_int32)])
+    _sig(hip, "trlm_gemm_keep_fp32", None, [C.c_void_p])
     _sig(hip, "trlm_gemm_force", C.c_int32, [C.c_void_p, C.c_char_p, C.c_int32])
     _sig(hip, "trlm_attn_job_table", C.c_int32, [C.c_uint32, C.c_uint32, C.c_uint32, C.c_uint32,
                                                  C.POINTER(C.c_int32)])
@@ -521,16 +524,26 @@ def _u32(a):
     return np.ascontiguousarray(a, np.uint32)
 
 
+def gemm_plan(ta, tb, M, N, K, batch=1, fp32=False, glu_F=0):
+    """(kernel, split-K factor) of trlm_gemm_plan_ex."""
+    sp = C.c_int32(0)
+    name = libs()[1].trlm_gemm_plan_ex(ta, tb, M, N, K, batch, fp32, glu_F, C.byref(sp))
+    return name.decode(), sp.value
+
+
 class Device:
     """A bare HIP context (kernel image loaded) with device-buffer helpers,
-    for exercising the GEMM and timing through the C ABI."""
+    for exercising the GEMM and timing through the C ABI.  fp32: its engine
+    keeps to the fp32 matrix cores (trlm_gemm_keep_fp32)."""
 
-    def __init__(self, image=KERNELS):
+    def __init__(self, image=KERNELS, fp32=False):
         _, hip = libs()
         self.hip = hip
         self.ctx = hip.hip_init(None, image.encode())
         hip.hip_set_current(C.byref(self.ctx))
         self.gemm = hip.trlm_gemm_create(C.byref(self.ctx))
+        if fp32:
+            hip.trlm_gemm_keep_fp32(self.gemm)
 
     def current(self):
         self.hip.hip_set_current(C.byref(self.ctx))
