@@ -339,7 +339,8 @@ def _probe(tmp_path, name, includes, flags):
     return subprocess.run([str(exe)], check=True, capture_output=True, text=True).stdout
 
 
-@pytest.mark.skipif(not os.path.isdir(REF), reason="reference tree not present")
+@pytest.mark.skipif(not os.path.isfile(os.path.join(REF, "model", "lm_model.c")),
+                    reason="the reference's sources are not present")
 def test_host_types_match_reference_headers(tmp_path):
     """sizeof and every field offset of the host types in trlm_host.h equal
     the reference's own definitions (runtime/types.h, runtime/memory.h,
@@ -354,7 +355,8 @@ def test_host_types_match_reference_headers(tmp_path):
     assert len(got.splitlines()) >= 50
 
 
-@pytest.mark.skipif(not os.path.isdir(REF), reason="reference tree not present")
+@pytest.mark.skipif(not os.path.isfile(os.path.join(REF, "model", "lm_model.c")),
+                    reason="the reference's sources are not present")
 def test_reference_programs_link_against_the_library(trlm):
     """oracle/dropin.sh: the reference's own programs, compiled against
     include/ as model/gpu_train.h, model/gpu_ops.h (+ hip_backend.h,
