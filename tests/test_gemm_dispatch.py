@@ -6,6 +6,8 @@ stand-ins of hip_backend.h's calls that write down what would be launched.
     both kinds of engine;
   - at most one 64x64 workgroup per CU (256) takes the fp32 tile, beyond it
     the split products;
+  - the gate/up product with its SwiGLU has the same lines: the small kernel,
+    the fp32 tile up to 256 workgroups, then the split products;
   - an engine kept to fp32 launches no split product."""
 import os
 import random
@@ -112,3 +114,16 @@ def test_lone_64x64_workgroups_take_the_fp32_tile(dispatch):
             assert kernel.startswith("k_gemm_" if lone else "k_xgemm_"), (call, launches)
             seen[lone] += 1
     assert min(seen.values()) >= 50, seen
+
+
+@pytest.mark.parametrize("M,F,K,want", [
+    (1, 32, 32, "k_smallgemm_nn_glu"), (100, 1024, 384, "k_smallgemm_nn_glu"), (256, 1024, 384, "k_smallgemm_nn_glu"),
+    (257, 1024, 384, "k_gemm_nn_64x64_k32_glu"), (512, 1024, 384, "k_gemm_nn_64x64_k32_glu"),
+    (513, 1024, 384, "k_xgemm_nn_64x64_k32_glu"), (8192, 1024, 384, "k_xgemm_nn_128x128_glu"),
+    (8192, 1056, 384, "k_xgemm_nn_64x64_k32_glu"), (64, 2048, 768, "k_smallgemm_nn_glu"),
+    (65, 2048, 768, "k_gemm_nn_64x64_k32_glu"), (64, 1024, 2048, "k_gemm_nn_64x64_k32_glu")])
+def test_swiglu_kernels(dispatch, M, F, K, want):
+    free, kept = dispatch([(fp32, 0, 0, M, 2 * F, K, F, 1, 0) for fp32 in (0, 1)])
+    tile = {"s": 32}.get(want[2], 128 if "128" in want else 64)
+    assert free[0] == [(want, -(-M // tile) * -(-2 * F // tile), 1)]
+    assert kept[0][0][0] == (want if "smallgemm" in want else "k_gemm_nn_64x64_k32_glu")

@@ -61,6 +61,7 @@ def test_through_the_trainer(trlm, orc, D, H, F, B, T):
     """Forward, loss and every gradient of a model whose layer products are
     all small (RoPE, SwiGLU with F a multiple of 32, bias gradients)."""
     V, L = 70, 2
+    assert trlm.gemm_plan(0, 0, B * T, 2 * F, D, fp32=True, glu_F=F) == ("k_smallgemm_nn_glu", 1)
     model = orc.Model(V, D, H, L, F)
     params = model.init(1337, 1)
     toks = orc.random_tokens(3000, V)

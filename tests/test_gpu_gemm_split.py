@@ -188,13 +188,17 @@ def test_values_without_a_split(dev, tile, ta, tb):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("F,B,T", [(64, 2, 70), (320, 3, 129), (1024, 8, 1024)])
-def test_swiglu_epilogue_of_both_tiles(trlm, orc, F, B, T):
+@pytest.mark.parametrize("F,B,T,kernel", [(32, 1, 33, "k_smallgemm_nn_glu"), (64, 2, 70, "k_smallgemm_nn_glu"),
+                                          (320, 3, 129, "k_gemm_nn_64x64_k32_glu"),
+                                          (1024, 2, 300, "k_xgemm_nn_64x64_k32_glu"),
+                                          (1024, 8, 1024, "k_xgemm_nn_128x128_glu")])
+def test_swiglu_epilogue_of_every_kernel(trlm, orc, F, B, T, kernel):
     """The gate/up product with the SwiGLU epilogue, through the decoder's
     prefill (whose engine takes the split products), at sizes where the plan
-    takes the 32-, the 64- and the 128-wide tile: the last position's logits
-    against the oracle's."""
+    takes the 32-, the fp32 64-, the split 64- and the 128-wide tile: the last
+    position's logits against the oracle's."""
     V, D, H, L = 150, 64, 2, 1
+    assert trlm.gemm_plan(0, 0, B * T, 2 * F, D, glu_F=F) == (kernel, 1)
     model = orc.Model(V, D, H, L, F)
     params = model.init(1337, 1)
     ids = orc.random_tokens(B * T, V, 4242, 13, hi_exclusive=V)

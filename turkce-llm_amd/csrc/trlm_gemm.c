@@ -422,13 +422,22 @@ static Plan make_plan(int layout, int M, int N, int K, u32 batch, const PlanOpts
     return p;
 }
 
-/* The plan of the gate/up product [M, 2F] with the SwiGLU epilogue: the
- * 128-wide tile where F holds whole half tiles and the plan model finds it
- * the faster of the two. */
+/* The plan of the gate/up product [M, 2F] with the SwiGLU epilogue.  MI355X,
+ * small / fp32 64x64 / split 64x64 / split 128x128 (us), K = 384, F = 1024:
+ * 100 rows (256 small tiles) 6.4 / 11.1 / 13.6 / 29, 256 rows (512) 10.1 / 11.4 / 13.8,
+ * 320 rows 14.4 / 11.7 / 13.9; K = 768, F = 2048: 64 rows (256) 12.3 / 18.3,
+ * 100 rows (512) 21.8 / 18.4 -- so one small tile per CU beyond 384 k.  At most one 64x64
+ * workgroup per CU takes the fp32 tile as in make_plan: 512 rows (256)
+ * 12.1 / 14.3, 768 rows (384) 18.6 / 16.9.  Beyond, the 128-wide tile where F
+ * holds whole half tiles and the plan model finds it the faster of the two. */
 static Plan make_glu_plan(int M, int F, int K, int fp32) {
     Plan p = { fp32 ? FP32 : SPLIT, T_64x64_K32, 1, K };
-    if (!fp32 && F % 64 == 0 &&
-        plan_cost(&PLAN_TILES[0], M, 2 * F, K, 1, 1) < plan_cost(&PLAN_TILES[2], M, 2 * F, K, 1, 1))
+    if (small_gemm(M, 2 * F, K, 1, 1) && (K <= 384 || (long long)cdiv(M, 32) * cdiv(2 * F, 32) <= CUS))
+        p.family = SMALL;
+    else if (tiles_of(p.tile, M, 2 * F, 1) <= CUS)
+        p.family = FP32;
+    else if (!fp32 && F % 64 == 0 &&
+             plan_cost(&PLAN_TILES[0], M, 2 * F, K, 1, 1) < plan_cost(&PLAN_TILES[2], M, 2 * F, K, 1, 1))
         p.tile = T_128x128;
     return p;
 }
@@ -509,11 +518,13 @@ i32 trlm_gemm_ws(TrlmGemm* e, i32 trans_a, i32 trans_b, hipDeviceptr_t A, hipDev
         p.M = M; p.N = N; p.K = K; p.lda = lda; p.ldb = ldb; p.ldc = ldc; p.ldr = ldr;
         p.splits = 1; p.kchunk = K; p.alpha = alpha; p.beta = 0.0f;
         const Plan pl = make_glu_plan(M, x->glu_F, K, e->fp32);
-        p.tiles_m = cdiv(M, TILES[pl.tile].bm); p.tiles_n = cdiv(N, TILES[pl.tile].bn);
+        const int tile = pl.family == SMALL ? 32 : TILES[pl.tile].bm;
+        p.tiles_m = cdiv(M, tile); p.tiles_n = cdiv(N, tile);
         p.glu_h = (float*)x->glu_h; p.glu_F = x->glu_F;
         plan_name(e->last, sizeof(e->last), &pl, L_NN, 1, 1);
         e->last_splits = 1;
-        launch(pl.family == FP32 ? e->glu : pl.tile == T_128x128 ? e->xglu128 : e->xglu, &p, 1);
+        launch(pl.family == SMALL ? e->small_glu : pl.family == FP32 ? e->glu : pl.tile == T_128x128 ? e->xglu128
+                                                                                                     : e->xglu, &p, 1);
         return 0;
     }
     if (csum && (batch != 1 || trans_b)) {
