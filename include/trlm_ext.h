@@ -59,9 +59,9 @@ void trlm_gemm(TrlmGemm* e, i32 trans_a, i32 trans_b, hipDeviceptr_t A, hipDevic
  * but the split-K partials go to a fixed 32 MiB scratch array that each GPU
  * holds from the first trlm_gemm_create on it until the process ends, so
  * the call allocates nothing.  A plan whose partials need more than 32 MiB
- * (splits x M x N floats; of the model's GEMMs only the full-size LM-head dX)
- * runs with the most splits whose partials fit, down to one split, which
- * needs none; its result then equals trlm_gemm on an engine forced to that
+ * (splits x M x N floats; of the 12-layer model's GEMMs at 8 x 1024 tokens the
+ * gate/up dX and dW, the down dW, and the LM head's dX and dW) runs with the
+ * most splits whose partials fit, down to one split, which needs none; its result then equals trlm_gemm on an engine forced to that
  * split count (trlm_gemm_force(e, NULL, splits)), and trlm_gemm_last_variant
  * reports it.  Returns 0; or -1, with a message on stderr and nothing
  * launched, when the engine's device is not the calling thread's current

@@ -8,6 +8,8 @@ stand-ins of hip_backend.h's calls that write down what would be launched.
     the split products;
   - the gate/up product with its SwiGLU has the same lines: the small kernel,
     the fp32 tile up to 256 workgroups, then the split products;
+  - with 32 MiB for the partials, as trlm_gemm_noalloc has, exactly the products
+    that its documentation names run with fewer splits than planned;
   - an engine kept to fp32 launches no split product."""
 import os
 import random
@@ -127,3 +129,21 @@ def test_swiglu_kernels(dispatch, M, F, K, want):
     tile = {"s": 32}.get(want[2], 128 if "128" in want else 64)
     assert free[0] == [(want, -(-M // tile) * -(-2 * F // tile), 1)]
     assert kept[0][0][0] == (want if "smallgemm" in want else "k_gemm_nn_64x64_k32_glu")
+
+
+def test_products_whose_partials_exceed_32_mib(dispatch):
+    N, D, F, V, room = 8192, 384, 1024, 31769, (32 << 20) // 4
+    shapes = {"QKV fwd": (0, 0, N, 3 * D, D), "out fwd": (0, 0, N, D, D), "gate/up fwd": (0, 0, N, 2 * F, D),
+              "down fwd": (0, 0, N, D, F), "head fwd": (0, 1, N, V, D), "QKV dX": (0, 1, N, D, 3 * D),
+              "out dX": (0, 1, N, D, D), "gate/up dX": (0, 1, N, D, 2 * F), "down dX": (0, 1, N, F, D),
+              "head dX": (0, 0, N, D, V), "QKV dW": (1, 0, D, 3 * D, N), "out dW": (1, 0, D, D, N),
+              "gate/up dW": (1, 0, D, 2 * F, N), "down dW": (1, 0, F, D, N), "head dW": (1, 0, V, D, N)}
+    fewer = set()
+    for (name, s), (_, (_, ran), (_, planned)) in zip(shapes.items(),
+                                                      dispatch([(0, *s, 0, 1, room) for s in shapes.values()])):
+        M, Nc = s[2], s[3]
+        assert ran == 1 or ran * M * Nc <= room, name
+        if ran < planned:
+            assert planned * M * Nc > room, name
+            fewer.add(name)
+    assert fewer == {"gate/up dX", "gate/up dW", "down dW", "head dX", "head dW"}
