@@ -10,7 +10,8 @@ stand-ins of hip_backend.h's calls that write down what would be launched.
     the fp32 tile up to 256 workgroups, then the split products;
   - with 32 MiB for the partials, as trlm_gemm_noalloc has, exactly the products
     that its documentation names run with fewer splits than planned;
-  - an engine kept to fp32 launches no split product."""
+  - an engine kept to fp32 launches no split product, and neither does any
+    engine for row statistics or column sums, which those kernels do not form."""
 import os
 import random
 import subprocess
@@ -38,16 +39,18 @@ int main(void) {
     memset(&ctx, 0, sizeof(ctx));
     TrlmGemm* e[2] = { trlm_gemm_create(&ctx), trlm_gemm_create(&ctx) };
     trlm_gemm_keep_fp32(e[1]);
-    int fp32, ta, tb, M, N, K, glu_F, aligned, splits;
+    int fp32, ta, tb, M, N, K, glu_F, aligned, splits, sums;
     unsigned long long ws;
-    while (scanf("%d %d %d %d %d %d %d %d %llu", &fp32, &ta, &tb, &M, &N, &K, &glu_F, &aligned, &ws) == 9) {
+    while (scanf("%d %d %d %d %d %d %d %d %llu %d", &fp32, &ta, &tb, &M, &N, &K, &glu_F, &aligned, &ws, &sums) == 10) {
         TrlmGemmExtra x;
         memset(&x, 0, sizeof(x));
+        if (sums && tb) { x.stats = (hipDeviceptr_t)0x800000; x.stats_cap = 1 << 20; }
+        if (sums && !tb) x.csum = (hipDeviceptr_t)0x900000;
         x.glu_h = glu_F ? (hipDeviceptr_t)0x600000 : NULL;
         x.glu_F = glu_F;
         const int la = ((ta ? M : K) + 3) / 4 * 4 + !aligned, lb = ((tb ? K : N) + 3) / 4 * 4 + !aligned;
         trlm_gemm_ws(e[fp32], ta, tb, (hipDeviceptr_t)0x100000, (hipDeviceptr_t)0x200000, (hipDeviceptr_t)0x300000,
-                     M, N, K, la, lb, N, 1, 0, 0, 0, 1.0f, 0.0f, NULL, NULL, N, glu_F ? &x : NULL,
+                     M, N, K, la, lb, N, 1, 0, 0, 0, 1.0f, 0.0f, NULL, NULL, N, glu_F || sums ? &x : NULL,
                      ws ? (hipDeviceptr_t)0x400000 : NULL, ws);
         const char* name = trlm_gemm_last_variant(e[fp32], &splits);
         printf("| %s %d ", name, splits);
@@ -61,7 +64,8 @@ int main(void) {
 
 @pytest.fixture(scope="module")
 def dispatch(tmp_path_factory):
-    """calls [(fp32, ta, tb, M, N, K, glu_F, aligned, fixed workspace floats)] ->
+    """calls [(fp32, ta, tb, M, N, K, glu_F, aligned, fixed workspace floats
+    [, row statistics (NT) or column sums])] ->
     [(launches [(kernel, grid x, grid z)], (reported, splits), (planned, splits))]"""
     d = tmp_path_factory.mktemp("dispatch")
     (d / "h.c").write_text(HARNESS)
@@ -72,7 +76,7 @@ def dispatch(tmp_path_factory):
                     "-lamdhip64"], check=True)
 
     def run(calls):
-        text = "\n".join(" ".join(str(int(v)) for v in c) for c in calls) + "\n"
+        text = "\n".join(" ".join(str(int(v)) for v in (*c, 0)[:10]) for c in calls) + "\n"
         out = subprocess.run([str(d / "h")], input=text, check=True, capture_output=True, text=True).stdout
         res = []
         for line in out.splitlines():
@@ -147,3 +151,10 @@ def test_products_whose_partials_exceed_32_mib(dispatch):
             assert planned * M * Nc > room, name
             fewer.add(name)
     assert fewer == {"gate/up dX", "gate/up dW", "down dW", "head dX", "head dW"}
+
+
+def test_sums_are_formed_by_the_fp32_kernels(dispatch):
+    calls = [(fp32, ta, tb, M, 2048, 8192, 0, aligned, 0, 1) for fp32 in (0, 1) for ta, tb in ((0, 1), (1, 0), (0, 0))
+             for M in (64, 384, 8192) for aligned in (0, 1)]
+    for call, (launches, (name, _), _) in zip(calls, dispatch(calls)):
+        assert name.startswith("k_gemm_") and launches[0][0] == name, call

@@ -596,7 +596,8 @@ __device__ __forceinline__ void gemm_store_lds(const GemmParams& p, float* C, co
     }
 }
 
-template <int BM, int BN, bool LDS_STORE = false, bool ILA = false, bool ILB = false>
+// STATS: the kernel is launched for row statistics too.
+template <int BM, int BN, bool LDS_STORE = false, bool ILA = false, bool ILB = false, bool STATS = true>
 __device__ __forceinline__ void gemm_epilogue(const GemmParams& p, float* C, const f32x16 (&acc)[BM / 64][BN / 64],
                                               int r0, int c0, int lane, float* lw = nullptr) {
     constexpr int FM = BM / 64, FN = BN / 64;
@@ -607,7 +608,7 @@ __device__ __forceinline__ void gemm_epilogue(const GemmParams& p, float* C, con
     auto row_of = [&](int i) { return ILA ? r0 + 2 * ml + i : r0 + i * 32 + ml; };
     // Row statistics: the NT layout only (the host refuses others), so never
     // with interleaved fragments
-    if constexpr (!ILA && !ILB) {
+    if constexpr (STATS && !ILA && !ILB) {
     if (p.stats) {
         // Row statistics for a softmax over the row (the LM head's
         // cross-entropy): per row, the max of this wave's BN/2 columns of

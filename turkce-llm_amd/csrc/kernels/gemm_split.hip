@@ -26,7 +26,8 @@
 // (1.6e-6).
 //
 // Serves raw GEMMs, the matmul node and the decoder's prefill; the trainer
-// keeps the fp32 tiles (trlm_gemm_keep_fp32), whose rounding its results pin.
+// keeps the fp32 tiles (trlm_gemm_keep_fp32), and with them the row statistics
+// and column sums that only it asks for: the host gives no such product here.
 //
 // Why: the fp32 matrix cores (157 TFLOP/s) were 79-86 % busy, so large GEMMs
 // could only gain from another unit.  Six bf16
@@ -323,11 +324,6 @@ __device__ __forceinline__ void gemm_x3_body(const GemmParams& p) {
     TileB tb;
     ta.init(A, p.lda, m0, p.M, kb);
     tb.init(B, p.ldb, n0, p.N, kb, GLU ? p.glu_F : 0);
-    const bool cs_on = TB == 0 && p.csum != nullptr && tm == 0;
-    constexpr int CW = TileB::NI * TileB::W;
-    float cs[CW];
-#pragma unroll
-    for (int i = 0; i < CW; i++) cs[i] = 0.f;
     // the partial k step (the last k) comes first, so the loop's loads need no checks
     const int rem = (ke - kb) % X3_BK, nk = (ke - kb) / X3_BK + (rem ? 1 : 0);
     if (rem) {
@@ -359,12 +355,6 @@ __device__ __forceinline__ void gemm_x3_body(const GemmParams& p) {
         }
         ta.store(la, scale);
         tb.store(lb, X3_SCALE);
-        if (TB == 0 && cs_on) {
-#pragma unroll
-            for (int i = 0; i < CW; i++)
-                cs[i] += ((tb.x[i][0] + tb.x[i][1]) + (tb.x[i][2] + tb.x[i][3])) +
-                         ((tb.x[i][4] + tb.x[i][5]) + (tb.x[i][6] + tb.x[i][7]));
-        }
         if (t + 1 < nk) {
             ta.load();
             tb.load();
@@ -388,23 +378,6 @@ __device__ __forceinline__ void gemm_x3_body(const GemmParams& p) {
         __syncthreads();
     }
     times(scale > 0.f ? X3_UNSCALE : -X3_UNSCALE);
-    if (TB == 0 && cs_on) {
-        // the four chunks' threads of a column, in chunk order
-        float* xs = (float*)lds;
-#pragma unroll
-        for (int i = 0; i < TileB::NI; i++) {
-            const int id = threadIdx.x + 256 * i;
-#pragma unroll
-            for (int w = 0; w < TileB::W; w++)
-                xs[(id / (BN / TileB::W)) * BN + TileB::W * (id % (BN / TileB::W)) + w] = cs[TileB::W * i + w];
-        }
-        __syncthreads();
-        if ((int)threadIdx.x < BN && n0 + (int)threadIdx.x < p.N) {
-            const int t = threadIdx.x;
-            float* dst = p.splits > 1 ? C + (long long)p.M * p.ldc : p.csum;
-            dst[n0 + t] = ((xs[t] + xs[BN + t]) + (xs[2 * BN + t] + xs[3 * BN + t]));
-        }
-    }
     // the largest magnitude (as bits) among the block's elements of C; what
     // an edge tile holds past M or N comes from padding and is left out
     unsigned top = 0;
@@ -444,7 +417,7 @@ __device__ __forceinline__ void gemm_x3_body(const GemmParams& p) {
         gemm_epilogue_glu2<BM, TileA::ILV>(p, acc, m0 + wm0, tn, wave, lane, (float*)lds);
     } else {
         constexpr bool LDS_STORE = 4 * 32 * (BN / 2) <= 4 * (TileA::UNITS + TileB::UNITS);
-        gemm_epilogue<BM, BN, LDS_STORE, TileA::ILV, TileB::ILV>(p, C, acc, m0 + wm0, n0 + wn0, lane,
+        gemm_epilogue<BM, BN, LDS_STORE, TileA::ILV, TileB::ILV, false>(p, C, acc, m0 + wm0, n0 + wn0, lane,
                                                                  (float*)lds + wave * 32 * (BN / 2));
     }
 }

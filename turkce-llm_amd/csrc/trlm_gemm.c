@@ -561,7 +561,8 @@ i32 trlm_gemm_ws(TrlmGemm* e, i32 trans_a, i32 trans_b, hipDeviceptr_t A, hipDev
     /* split-K: raw partials into the workspace, then an ordered reduction;
      * with column sums each split's slab has one more row, M, for them */
     const u64 slab = ((u64)M + (csum ? 1u : 0u)) * (u64)N;
-    const PlanOpts o = { aligned, e->fp32, stats != NULL, stats || rope, e->force_tile, e->force_splits, slab,
+    /* row statistics and column sums are the fp32 kernels' */
+    const PlanOpts o = { aligned, e->fp32 || stats || csum, stats != NULL, stats || rope, e->force_tile, e->force_splits, slab,
                          fixed_ws ? fixed_floats : ANY_ROOM };
     const Plan pl = make_plan(layout, M, N, K, batch, &o);
     const int tile = pl.tile, splits = pl.splits;
