@@ -1,7 +1,8 @@
 """hip_h2d, hip_d2h and hip_d2h_rows: bytes arrive whole at every edge of the
 staging (small copies up to 128 KiB, downloads from 2 MiB on in 4 MiB blocks
-with 512 KiB to a thread), rows lose their padding, and threads that share one
-context do not mix their bytes."""
+with 512 KiB to a thread), rows lose their padding, pinned memory is a copy's
+own source and destination, and threads that share one context do not mix
+their bytes."""
 import ctypes as C
 import threading
 
@@ -57,6 +58,28 @@ def test_rows(dev, row_bytes, pitch, rows):
     want = [x[r * pitch:r * pitch + row_bytes] for r in range(rows)]
     assert np.array_equal(got[:rows * row_bytes], np.concatenate(want) if want else got[:0])
     assert (got[rows * row_bytes:] == 7).all()
+
+
+@pytest.mark.parametrize("row_bytes,pitch,rows", [(4096, 4096, 1), (4, 16, 5), (31769 * 4, 31772 * 4, 34),
+                                                  (4 * MB + 5, 4 * MB + 16, 2)])
+def test_pinned_memory(dev, row_bytes, pitch, rows):
+    import torch
+    dev.current()
+    fn = dev.hip.hip_d2h_rows
+    fn.argtypes, fn.restype = [C.c_void_p, C.c_void_p, C.c_uint64, C.c_uint64, C.c_uint64], None
+    n = (rows - 1) * pitch + row_bytes
+    a, b = [torch.empty(n + 64, dtype=torch.uint8, pin_memory=True).numpy() for _ in range(2)]
+    a[:n] = np.random.default_rng(rows).integers(0, 256, n, np.uint8)
+    p = dev.empty(n)
+    dev.hip.hip_h2d(p, a.ctypes.data, n)
+    b[:] = 7
+    dev.hip.hip_d2h(b.ctypes.data, p, n)
+    assert np.array_equal(a[:n], b[:n]) and (b[n:] == 7).all()
+    b[:] = 7
+    fn(b.ctypes.data, p, pitch, row_bytes, rows)
+    dev.free(p)
+    assert np.array_equal(b[:rows * row_bytes], np.concatenate([a[r * pitch:r * pitch + row_bytes] for r in range(rows)]))
+    assert (b[rows * row_bytes:] == 7).all()
 
 
 def test_threads_share_a_context(dev):
