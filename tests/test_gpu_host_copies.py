@@ -63,12 +63,16 @@ def test_rows(dev, row_bytes, pitch, rows):
 @pytest.mark.parametrize("row_bytes,pitch,rows", [(4096, 4096, 1), (4, 16, 5), (31769 * 4, 31772 * 4, 34),
                                                   (4 * MB + 5, 4 * MB + 16, 2)])
 def test_pinned_memory(dev, row_bytes, pitch, rows):
-    import torch
     dev.current()
+    with open("/proc/self/maps") as fh:     # the HIP runtime that libtrlm_hip.so loaded
+        hip = C.CDLL(sorted({line.split()[-1] for line in fh if "libamdhip64.so" in line})[0])
     fn = dev.hip.hip_d2h_rows
     fn.argtypes, fn.restype = [C.c_void_p, C.c_void_p, C.c_uint64, C.c_uint64, C.c_uint64], None
     n = (rows - 1) * pitch + row_bytes
-    a, b = [torch.empty(n + 64, dtype=torch.uint8, pin_memory=True).numpy() for _ in range(2)]
+    mem = [C.c_void_p() for _ in range(2)]
+    for m in mem:
+        assert hip.hipHostMalloc(C.byref(m), C.c_size_t(n + 64), C.c_uint(0)) == 0
+    a, b = [np.ctypeslib.as_array(C.cast(m, C.POINTER(C.c_uint8)), (n + 64,)) for m in mem]
     a[:n] = np.random.default_rng(rows).integers(0, 256, n, np.uint8)
     p = dev.empty(n)
     dev.hip.hip_h2d(p, a.ctypes.data, n)
@@ -80,6 +84,8 @@ def test_pinned_memory(dev, row_bytes, pitch, rows):
     dev.free(p)
     assert np.array_equal(b[:rows * row_bytes], np.concatenate([a[r * pitch:r * pitch + row_bytes] for r in range(rows)]))
     assert (b[rows * row_bytes:] == 7).all()
+    for m in mem:
+        assert hip.hipHostFree(m) == 0
 
 
 def test_threads_share_a_context(dev):
