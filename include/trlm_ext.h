@@ -125,8 +125,9 @@ bool32 gpu_trainer_checkpoint_load(GpuTrainer* g, const char* path, Node** param
 
 /* ---- KV-cache decode (generate.c:57-73,186-212 without the per-step
  * full-window recompute).  The decoder uses the trainer's resident
- * parameters, kernels, stream and GEMM engine; it owns a K/V cache of
- * L x batch x H x max_ctx x hd floats each.  All sequences of a batch share
+ * parameters, kernels and stream; it owns a K/V cache of
+ * L x batch x H x max_ctx x hd floats each, and the prefill's GEMM engine,
+ * which is not kept to fp32.  All sequences of a batch share
  * one length.  Errors (tokens outside the vocabulary, a full context, a step
  * before the prefill) print "[HIP ERROR] gpu_decode: ..." and _exit(1). */
 typedef struct TrlmDecoder TrlmDecoder;

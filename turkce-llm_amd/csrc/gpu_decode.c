@@ -43,7 +43,7 @@
 
 struct TrlmDecoder {
     GpuTrainer* g;
-    TrlmGemm* gemm;                     /* the prefill's products (made at the first prefill) */
+    TrlmGemm* gemm;                     /* the prefill's products (the trainer's engines keep to fp32) */
     u32 B, ctx, len;
     u32 L, H, hd, D, F, V, ldv;
     f32 scale;
@@ -157,6 +157,7 @@ TrlmDecoder* gpu_decoder_create(GpuTrainer* g, u32 batch, u32 max_ctx) {
     d->k_head = hip_get_kernel(c, g->D <= 128 ? "k_dec_head_k8" : g->D <= 384 ? "k_dec_head_k24" : "k_dec_head_k32");
     snprintf(name, sizeof(name), "k_dec_qkv_attn_hd%u", g->hd);
     d->k_qkv_attn = hip_get_kernel(c, name);
+    d->gemm = trlm_gemm_create(c);
     d->pos_dev = hip_alloc(sizeof(i32));
     hip_sync();
     return d;
@@ -244,10 +245,9 @@ void gpu_decoder_prefill(TrlmDecoder* d, const u32* ids, u32 len) {
         d->pre_rows = R;
     }
     /* The trainer's forward on batch x len rows: a copy of the trainer with
-     * the same parameters and kernels, whose activations are one
-     * set of buffers shared by every layer (nothing is kept for a backward). */
+     * the same parameters and kernels, whose activations are one set of
+     * buffers shared by every layer (nothing is kept for a backward). */
     GpuTrainer pf = *g;
-    if (!d->gemm) d->gemm = trlm_gemm_create(&g->hip);   /* not the trainer's, which keeps to fp32 tiles */
     pf.gemm = d->gemm;
     pf.B = d->B; pf.T = len; pf.N = (u32)R;
     for (u32 l = 0; l < g->L; l++) {

@@ -81,6 +81,10 @@ i32 trlm_gemm_ws(TrlmGemm* e, i32 trans_a, i32 trans_b, hipDeviceptr_t A, hipDev
                  i32 M, i32 N, i32 K, i32 lda, i32 ldb, i32 ldc, u32 batch, i64 sA, i64 sB, i64 sC,
                  f32 alpha, f32 beta, hipDeviceptr_t bias, hipDeviceptr_t resid, i32 ldr, const TrlmGemmExtra* x,
                  hipDeviceptr_t fixed_ws, u64 fixed_floats);
+/* An engine kept to fp32 (trlm_gemm_keep_fp32) from the start: it does not
+ * look up the split products' kernels (0.7-1.7 us each; a trainer makes its two
+ * engines in its first pass). */
+TrlmGemm* trlm_gemm_create_fp32(HipCtx* ctx);
 /* The device of the context the engine was created in. */
 i32 trlm_gemm_device(const TrlmGemm* e);
 /* noalloc.hip: resolves the device address of the GEMM scratch array on

@@ -396,14 +396,8 @@ GpuTrainer gpu_trainer_create(Allocator* alloc, const char* ptx_path, const LMMo
  * is returned by value, so the engine is bound lazily on first use. */
 static void bind(GpuTrainer* g) {
     hip_set_current(&g->hip);
-    if (!g->gemm) {
-        g->gemm = trlm_gemm_create(&g->hip);
-        trlm_gemm_keep_fp32(g->gemm);
-    }
-    if (!g->gemm_side) {
-        g->gemm_side = trlm_gemm_create(&g->hip);
-        trlm_gemm_keep_fp32(g->gemm_side);
-    }
+    if (!g->gemm) g->gemm = trlm_gemm_create_fp32(&g->hip);
+    if (!g->gemm_side) g->gemm_side = trlm_gemm_create_fp32(&g->hip);
 }
 
 void gpu_trainer_destroy(GpuTrainer* g) {

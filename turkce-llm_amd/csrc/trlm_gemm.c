@@ -67,22 +67,24 @@ struct TrlmGemm {
     i32 force_splits;  /* 0: automatic split-K */
 };
 
-TrlmGemm* trlm_gemm_create(HipCtx* ctx) {
+static TrlmGemm* create(HipCtx* ctx, int fp32) {
     TrlmGemm* e = (TrlmGemm*)calloc(1, sizeof(TrlmGemm));
     e->ctx = ctx;
     e->force_tile = -1;
+    e->fp32 = fp32;
     char name[64];
     for (int l = 0; l < 3; l++)
         for (int t = 0; t < T_COUNT; t++) {
             snprintf(name, sizeof(name), "k_gemm_%s_%s", LAYOUT_NAME[l], TILES[t].name);
             e->k[l][t] = hip_get_kernel(ctx, name);
-            if (!has_split(t)) continue;
+            if (fp32 || !has_split(t)) continue;
             snprintf(name, sizeof(name), "k_xgemm_%s_%s", LAYOUT_NAME[l], TILES[t].name);
             e->x[l][t] = hip_get_kernel(ctx, name);
         }
     for (int l = 0; l < 4; l++) {
         snprintf(name, sizeof(name), "k_gemm_%s_64x64_u", LAYOUT_NAME[l]);
         e->ku[l] = hip_get_kernel(ctx, name);
+        if (fp32) continue;
         snprintf(name, sizeof(name), "k_xgemm_%s_64x64_u", LAYOUT_NAME[l]);
         e->xu[l] = hip_get_kernel(ctx, name);
         if (l == 3) break;
@@ -99,11 +101,17 @@ TrlmGemm* trlm_gemm_create(HipCtx* ctx) {
     e->reduce = hip_get_kernel(ctx, "k_gemm_splitk_reduce");
     e->reduce4 = hip_get_kernel(ctx, "k_gemm_splitk_reduce4");
     e->glu = hip_get_kernel(ctx, "k_gemm_nn_64x64_k32_glu");
-    e->xglu = hip_get_kernel(ctx, "k_xgemm_nn_64x64_k32_glu");
-    e->xglu128 = hip_get_kernel(ctx, "k_xgemm_nn_128x128_glu");
+    if (!fp32) {
+        e->xglu = hip_get_kernel(ctx, "k_xgemm_nn_64x64_k32_glu");
+        e->xglu128 = hip_get_kernel(ctx, "k_xgemm_nn_128x128_glu");
+    }
     trlm_noalloc_setup(ctx->device);
     return e;
 }
+
+TrlmGemm* trlm_gemm_create(HipCtx* ctx) { return create(ctx, 0); }
+
+TrlmGemm* trlm_gemm_create_fp32(HipCtx* ctx) { return create(ctx, 1); }
 
 /* The engine's products keep to the fp32 matrix cores, with the tiles and
  * split-K of the fp32 plan (products of few tiles take k_smallgemm_*, which is
