@@ -651,7 +651,7 @@ def traffic_summarize(fetch_dir, write_dir):
                 if r["Counter_Name"] != counter:
                     continue
                 k = "copy" if "copyBuffer" in r["Kernel_Name"] else (
-                    "head" if r["Kernel_Name"].startswith("k_gemm_nt") else None)
+                    "head" if r["Kernel_Name"].startswith(("k_gemm_nt", "k_xgemm_nt")) else None)
                 if k:
                     vals.setdefault(k, {}).setdefault(r["Dispatch_Id"], 0.0)
                     vals[k][r["Dispatch_Id"]] += float(r["Counter_Value"])
